@@ -20,12 +20,12 @@ LIB = os.path.join(LIBDIR, "libgllm_attn.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["paged_attention.hip", "paged_attention_f16.hip", "api.hip", "rope_kv_write.hip", "attention_f32.hip",
-           "metadata.hip", "qkv_proj.hip"]
-NO_CONTRACT = {"rope_kv_write.hip", "attention_f32.hip", "qkv_proj.hip"}
+SOURCES = ["paged_attention.hip", "paged_attention_f16.hip", "api.hip", "rope_kv_write.hip", "generic_attention.hip",
+           "generic_attention_bf16.hip", "generic_attention_f16.hip", "metadata.hip", "qkv_proj.hip"]
+GENERIC = {"generic_attention.hip", "generic_attention_bf16.hip", "generic_attention_f16.hip"}
+NO_CONTRACT = {"rope_kv_write.hip", "qkv_proj.hip"} | GENERIC
 # MFMA accumulators stay in VGPRs (no per-tile AGPR<->VGPR copies)
-EXTRA = {"paged_attention.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
-         "paged_attention_f16.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"]}
+EXTRA = {f: ["-mllvm", "--amdgpu-mfma-vgpr-form"] for f in {"paged_attention.hip", "paged_attention_f16.hip"} | GENERIC}
 COMMON = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # packed fp32 VALU ops are disabled on purpose for every HIP unit

@@ -182,7 +182,10 @@ struct gllm_attn_plan {
   int64_t total_rows = 0;
   int64_t n_partials = 0;
   std::vector<SeqInfo> seqs;
-  std::vector<WorkItem> items;
+  std::vector<WorkItem> items;   // MFMA kernels; generic plans: the tiled kernel's
+  // generic kernels: query rows from which a sequence is tiled (0: none), the
+  // largest query length below that
+  int32_t tile_min_q = 0, max_stream_q = 0;
   // page-balanced decode: workgroup w runs segs[seg_ptr[w] .. seg_ptr[w + 1])
   std::vector<DecodeSeg> segs;
   std::vector<int32_t> seg_ptr;
@@ -630,7 +633,7 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
   p->num_seqs = num_seqs; p->Hq = num_q_heads; p->Hkv = num_kv_heads; p->D = head_dim;
   p->bs = block_size; p->dtype = dtype; p->mfma = mfma;
   p->seqs.resize(num_seqs);
-  int64_t row = 0, decode_tokens = 0;
+  int64_t row = 0, decode_tokens = 0, tile_wgs = 0;
   for (int i = 0; i < num_seqs; ++i) {
     const int32_t ql = query_lens[i], sl = seq_lens[i];
     if (ql < 1 || sl < ql) {
@@ -648,6 +651,8 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     s.q_len = ql;
     row += ql;
     p->max_q = std::max(p->max_q, ql);
+    if (ql < kTileMinRows) p->max_stream_q = std::max(p->max_stream_q, ql);
+    else tile_wgs += ((int64_t)ql * G + kTileCols - 1) / kTileCols * num_kv_heads;
     if (mfma && ql * G <= 16) decode_tokens += sl;
   }
   p->total_rows = q_seq_stride > 0 ? (int64_t)num_seqs * q_seq_stride : row;
@@ -655,6 +660,9 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     delete p;
     return fail(GLLM_ATTN_EINVAL, "too many query rows");
   }
+
+  if (tile_wgs >= kTileMinWgs) p->tile_min_q = kTileMinRows;
+  else p->max_stream_q = p->max_q;
 
   if (mfma) {
     const int cus = device_cus();
@@ -832,6 +840,29 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     }
     }
   }
+  if (!mfma && p->tile_min_q > 0) {
+    // Generic plan: one item per kTileCols (query row, head) columns of a kv
+    // head of every sequence the tiled kernel takes, most keys first.
+    struct Keyed { int64_t kend; WorkItem it; };
+    std::vector<Keyed> tiles;
+    for (int i = 0; i < num_seqs; ++i) {
+      const SeqInfo& s = p->seqs[i];
+      if (s.q_len < p->tile_min_q) continue;
+      const int64_t ncol = (int64_t)s.q_len * G;
+      for (int64_t w = 0; w * kTileCols < ncol; ++w) {
+        const int64_t kend = s.ctx_len + (std::min((w + 1) * kTileCols, ncol) - 1) / G + 1;
+        for (int h = 0; h < num_kv_heads; ++h)
+          tiles.push_back({kend, WorkItem{(int32_t)(w << 8), i, h, s.q_row_start, s.ctx_len, s.q_len, 0, 0}});
+      }
+    }
+    std::stable_sort(tiles.begin(), tiles.end(), [](const Keyed& x, const Keyed& y) { return x.kend > y.kend; });
+    if (tiles.size() > (size_t)INT32_MAX) {
+      delete p;
+      return fail(GLLM_ATTN_EINVAL, "too many work items");
+    }
+    p->items.reserve(tiles.size());
+    for (const Keyed& k : tiles) p->items.push_back(k.it);
+  }
   if (p->n_partials > (int64_t)INT32_MAX / 16) {
     delete p;
     return fail(GLLM_ATTN_EINVAL, "too many split partials");
@@ -998,7 +1029,12 @@ static int paged_attention_impl(const gllm_attn_plan* p, const void* q, int64_t 
   if (use_mfma)
     return hip_check(launch_paged_attention_mfma(a, p->n_prefill_seqs > 0, p->n_decode_seqs > 0, st),
                      "paged attention launch");
-  return hip_check(launch_attention_f32(a, false, p->num_seqs, p->max_q, st), "generic attention launch");
+  a.tile_min_q = p->tile_min_q;
+  if (!p->mfma) {
+    a.tile_items = a.items;
+    a.n_tile_items = a.n_items;
+  }
+  return hip_check(launch_attention_generic(a, false, p->num_seqs, p->max_q, p->max_stream_q, st), "generic attention launch");
 }
 
 int gllm_paged_attention(const gllm_attn_plan* p, const void* q, int64_t q_row_stride, void* out,
@@ -1058,7 +1094,7 @@ int gllm_attention_dense(const void* q, int64_t q_row_stride, const void* k, int
   hipStream_t st = (hipStream_t)stream;
   if (mfma_dtype(dtype) && (head_dim == 64 || head_dim == 128))
     return hip_check(launch_dense_attention_mfma(a, batch, q_len, st), "dense attention launch");
-  return hip_check(launch_attention_f32(a, true, batch, q_len, st), "generic dense attention launch");
+  return hip_check(launch_attention_generic(a, true, batch, q_len, q_len, st), "generic dense attention launch");
 }
 
 }  // extern "C"

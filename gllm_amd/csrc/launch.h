@@ -39,6 +39,20 @@ enum : int32_t { kRopeNone = 0, kRopeByPosition = 1, kRopeByRow = 2 };
 constexpr int kPrefillOnlyWaves = 8;
 constexpr int kPrefillOnlyStages = 4;
 
+// Generic attention: (query row, head) columns of one workgroup of the stream
+// kernel (attention_stream.h) and of the tiled kernel (attention_tile.h); the
+// tiled one takes the sequences of at least kTileMinRows query rows when they
+// make at least kTileMinWgs of its workgroups: below that it leaves CUs idle
+// and walks a sequence's keys in one wave each, where the stream kernel splits
+// them over eight.  Measured (stream / tile us, 32 / 8 heads, 2048 cached
+// keys): 64 workgroups (1 x 256 rows) 80 / 234 at D = 64, 134 / 381 at D = 128;
+// 128 (8 x 64) 150 / 220 and 243 / 358; 256 (32 x 32) 348 / 222 and 609 / 372;
+// 512 (8 x 256) 593 / 383 and 1000 / 657.
+constexpr int kStreamCols = 16;
+constexpr int kTileCols = 128;
+constexpr int kTileMinRows = 17;
+constexpr int kTileMinWgs = 192;
+
 // Paged attention (decode / prefill / mixed) and the dense-bias op share it.
 struct AttnArgs {
   const void* q;             // query rows, heads at h*D within a row
@@ -97,6 +111,13 @@ struct AttnArgs {
   const void* k_new;
   const void* v_new;
   int64_t k_new_row_stride, v_new_row_stride;
+  // generic kernels: sequences of at least tile_min_q query rows run on the
+  // tiled kernel (0: none), the others on the stream kernel
+  const WorkItem* tile_items;  // the tiled kernel's work (null: a grid over every sequence)
+  int32_t n_tile_items;
+  int32_t tile_min_q;
+  int32_t vec_rows;            // K/V rows aligned for the kernel's vector loads (set by the launcher)
+  int32_t vec_out;             // output rows aligned for stores of 4 elements (set by the launcher)
 };
 
 struct MetadataArgs {
@@ -157,7 +178,9 @@ hipError_t launch_build_metadata(const MetadataArgs& a, hipStream_t stream);
 // the model dtype or fp8 e4m3fn
 hipError_t launch_paged_attention_mfma(const AttnArgs& a, bool has_prefill, bool has_decode, hipStream_t stream);
 hipError_t launch_dense_attention_mfma(const AttnArgs& a, int B, int Tq, hipStream_t stream);
-hipError_t launch_attention_f32(const AttnArgs& a, bool dense, int B, int max_q, hipStream_t stream);
+// Generic kernels: max_q the largest query length, max_stream_q the largest of
+// the sequences on the stream kernel (0: every sequence is tiled)
+hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, hipStream_t stream);
 hipError_t launch_fill_zero_i32(int32_t* p, int64_t n, hipStream_t stream);
 
 }  // namespace gllm

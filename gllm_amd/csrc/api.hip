@@ -1091,6 +1091,7 @@ int gllm_attention_dense(const void* q, int64_t q_row_stride, const void* k, int
   a.v_batch_stride = v_batch_stride; a.v_row_stride = v_row_stride;
   a.bias = bias; a.bias_batch_stride = bias_batch_stride; a.bias_row_stride = bias_row_stride;
   a.dense_T = kv_len; a.dense_Tq = q_len;
+  a.bias_vec = ((uintptr_t)bias & 7) == 0 && bias_batch_stride % 4 == 0 && bias_row_stride % 4 == 0 && kv_len % 4 == 0;
   hipStream_t st = (hipStream_t)stream;
   if (mfma_dtype(dtype) && (head_dim == 64 || head_dim == 128))
     return hip_check(launch_dense_attention_mfma(a, batch, q_len, st), "dense attention launch");

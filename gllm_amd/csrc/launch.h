@@ -75,6 +75,7 @@ struct AttnArgs {
   int64_t k_batch_stride, k_row_stride, v_batch_stride, v_row_stride;
   const void* bias;           // [B, T_q, T] model dtype
   int64_t bias_batch_stride, bias_row_stride;
+  int32_t bias_vec;           // rows 4-element aligned and dense_T a multiple of 4: 8-byte bias loads
   int32_t dense_T;            // keys per batch entry
   int32_t dense_Tq;           // query rows per batch entry (q/out row = b * dense_Tq + r)
   // rope applied to q on load

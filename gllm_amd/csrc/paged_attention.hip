@@ -623,17 +623,25 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
     qstart = it.q_row_start;
   }
   const int G = a.num_q_heads / a.num_kv_heads;
-  const int nrb = (qlen + 31) / 32;
+  // The wave's 32 MFMA columns.  Paged: 32 query rows of one head (the causal
+  // edge then cuts few tiles).  Dense: neighbouring (row, head of the group)
+  // pairs, so the G heads of a row read its bias together and a wave touches
+  // 32 / G bias rows instead of 32 (those loads bound the op otherwise: batch 8,
+  // 512 rows, 1024 keys, 32 / 8 heads of 64 267 us with two-byte loads of 32
+  // rows per wave, 73 with this and 8-byte loads a tile ahead).
   const int combo = wgrp * NW + wave;
-  const bool wact = combo < G * nrb;
-  const int g = wact ? combo % G : 0;
-  const int rblk = wact ? combo / G : 0;
+  const int nrb = (qlen + 31) / 32;
+  const int ncol = qlen * G;                // dense
+  const bool wact = DENSE ? combo * 32 < ncol : combo < G * nrb;
+  const int dcol = min(combo * 32 + n, ncol - 1);
+  const int g = DENSE ? dcol % G : (wact ? combo % G : 0);
+  const int rblk = !DENSE && wact ? combo / G : 0;
   const int r0 = rblk * 32;
   const int last_combo = min(wgrp * NW + NW - 1, G * nrb - 1);
   const int kend_wg = DENSE ? TK : ctx + min(qlen - 1, (last_combo / G) * 32 + 31) + 1;
   const int kend_w = DENSE ? TK : ctx + min(qlen - 1, r0 + 31) + 1;
-  const int r = r0 + n;
-  const bool row_ok = wact && r < qlen;
+  const int r = DENSE ? dcol / G : r0 + n;
+  const bool row_ok = wact && (DENSE ? combo * 32 + n < ncol : r < qlen);
   const int rr = min(r, qlen - 1);
   const int vis = ctx + rr;
   const int64_t qrow = qstart + rr;
@@ -851,15 +859,47 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
       }
     }
   };
-  auto sm_max = [&](f32x16& s, int k0, bool mask, Soft& q) {
-    if (DENSE) {
-      const T* bp = (const T*)a.bias + (int64_t)seq * a.bias_batch_stride + (int64_t)rr * a.bias_row_stride;
+  // Dense: the bias of a tile's two halves, loaded a tile ahead (at D = 128, where
+  // registers are short, at the tile's start, under its QK MFMAs); four keys
+  // per 8-byte load where the rows are aligned and T is a multiple of 4, other
+  // biases element by element.
+  constexpr bool kBiasAhead = D == 64;
+  const T* const bp = DENSE ? (const T*)a.bias + (int64_t)seq * a.bias_batch_stride + (int64_t)rr * a.bias_row_stride
+                            : nullptr;
+  u32x2 bcur[DENSE ? 2 : 1][4], bnext[DENSE ? 2 : 1][4];
+  auto bias_load = [&](int ts) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {   // bias in natural-log units: to log2 units like the scaled scores
-        const int key = k0 + 8 * (j >> 2) + 4 * h + (j & 3);
-        const float bv = key < TK ? (float)bp[key] : kNegInf;
-        s[j] = __builtin_fmaf(s[j], sl2, __builtin_fmaf(bv, kLog2e, sbase));
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {
+        const int key = ts + 32 * kb + 8 * jq + 4 * h;
+        if (a.bias_vec) {
+          bnext[kb][jq] = *reinterpret_cast<const u32x2*>(bp + min(key, TK - 4));
+        } else {
+          const uint16_t* b16 = reinterpret_cast<const uint16_t*>(bp);
+          uint32_t w[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = b16[min(key + e, TK - 1)];
+          bnext[kb][jq] = u32x2{w[0] | (w[1] << 16), w[2] | (w[3] << 16)};
+        }
       }
+  };
+  auto sm_max = [&](f32x16& s, int k0, bool mask, Soft& q, const u32x2* bw) {
+    if (DENSE) {
+      float bv[16];
+#pragma unroll
+      for (int j = 0; j < 16; j += 2) {
+        const uint32_t w = bw[j >> 2][(j >> 1) & 1];
+        bv[j] = E16<T>::lo(w);
+        bv[j + 1] = E16<T>::hi(w);
+      }
+      if (k0 + 32 > TK) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) bv[j] = k0 + 8 * (j >> 2) + 4 * h + (j & 3) < TK ? bv[j] : kNegInf;
+      }
+#pragma unroll
+      for (int j = 0; j < 16; ++j)   // bias in natural-log units: to log2 units like the scaled scores
+        s[j] = __builtin_fmaf(s[j], sl2, __builtin_fmaf(bv[j], kLog2e, sbase));
     } else if (mask) {
       apply_mask(s, k0);
     }
@@ -901,10 +941,10 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
   };
   // Logical softmax piece p (0..7) of a half: max (dense) or prep (paged),
   // 4 x exp, convert, sum.
-  auto sm_piece = [&](int p, f32x16& s, int k0, bool mask, Soft& q, u32x4* pb, bool first) {
+  auto sm_piece = [&](int p, f32x16& s, int kb, int k0, bool mask, Soft& q, u32x4* pb, bool first) {
     if (p == 0) {
       if (kFast) fs_prep(s, k0, mask, first);
-      else sm_max(s, k0, mask, q);
+      else sm_max(s, k0, mask, q, bcur[DENSE ? kb : 0]);
     }
     else if (p <= 4) sm_exp(s, 4 * (p - 1));
     else if (p == 5) sm_cvt(s, pb);
@@ -987,7 +1027,15 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
     for (int kk = 0; kk < NQ; ++kk) ka[0][kk] = *reinterpret_cast<const u32x4*>(st + koff[kk]);
     s0 = f32x16{};
     s1 = f32x16{};
-    if (!kFast) sbase = m == kNegInf ? 0.f : -m;   // both halves start from the max before this tile
+    if (!kFast) {
+      sbase = m == kNegInf ? 0.f : -m;   // both halves start from the max before this tile
+      if (DENSE && !kBiasAhead) bias_load(ts);
+#pragma unroll
+      for (int kb = 0; kb < (DENSE ? 2 : 1); ++kb)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) bcur[kb][jq] = bnext[kb][jq];
+      if (DENSE && kBiasAhead) bias_load(min(ts + BN, (TK - 1) / BN * BN));   // the next tile's
+    }
     // K of half 1 is read between the MFMAs of half 0: the eight waves' reads
     // after a barrier do not all hit LDS at once, and fewer registers are live
 #pragma unroll
@@ -1008,7 +1056,7 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int p = kk * 8 / NQ; p < (kk + 1) * 8 / NQ; ++p) sm_piece(p, s0, ts, mask, q0, pb0, first);
+      for (int p = kk * 8 / NQ; p < (kk + 1) * 8 / NQ; ++p) sm_piece(p, s0, 0, ts, mask, q0, pb0, first);
       __builtin_amdgcn_sched_barrier(0);
     }
     commit(q0, st, 0, ts, mask, pb0);
@@ -1021,7 +1069,7 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int p = i * 8 / (2 * NO); p < (i + 1) * 8 / (2 * NO); ++p)
-        sm_piece(p, s1, ts + 32, mask, q1, pb1, false);
+        sm_piece(p, s1, 1, ts + 32, mask, q1, pb1, false);
       __builtin_amdgcn_sched_barrier(0);
     }
     commit(q1, st, 1, ts + 32, mask, pb1);
@@ -1097,6 +1145,7 @@ __device__ __forceinline__ void prefill_wg(const AttnArgs& a, const WorkItem& it
       if (tid + k * NT < nbc) lbid[tid + k * NT] = lb[k] < (uint64_t)a.num_blocks ? (int32_t)lb[k] : 0;
   }
   uint32_t nbid[CHD];
+  if (DENSE && kBiasAhead && wact) bias_load(0);
 
   // Q as the B operand of S^T = K Q^T: lane holds Q[row n][16kk + 8h + i].
   {
@@ -1376,7 +1425,7 @@ hipError_t launch_paged_attention_mfma(const AttnArgs& a, bool has_prefill, bool
 
 hipError_t launch_dense_attention_mfma(const AttnArgs& a, int B, int Tq, hipStream_t st) {
   const int G = a.num_q_heads / a.num_kv_heads;
-  const int nwg = (G * ((Tq + 31) / 32) + kWaves - 1) / kWaves;
+  const int nwg = (int)(((int64_t)G * Tq + 32 * kWaves - 1) / (32 * kWaves));
   const int64_t blocks = (int64_t)B * a.num_kv_heads * nwg;
   if (blocks == 0) return hipSuccess;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;

@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <new>
 #include <string>
@@ -189,11 +190,13 @@ struct gllm_attn_plan {
   // page-balanced decode: workgroup w runs segs[seg_ptr[w] .. seg_ptr[w + 1])
   std::vector<DecodeSeg> segs;
   std::vector<int32_t> seg_ptr;
+  std::vector<MergeInfo> merge;  // [num_seqs * head_groups], plans with partials
+  int32_t head_groups = 1;
   // staging copy of [items | seqs] in pinned host memory (from the pool), device offsets
   void* pinned = nullptr;
   size_t pinned_cap = 0;
   bool pinned_is_host_malloc = false;  // hipHostMalloc unavailable (no device): plain malloc
-  size_t off_items = 0, off_seqs = 0, off_segs = 0, off_segptr = 0, off_ctr = 0, off_ml = 0, off_part = 0, ws_bytes = 0;
+  size_t off_items = 0, off_seqs = 0, off_segs = 0, off_segptr = 0, off_merge = 0, off_ml = 0, off_part = 0, ws_bytes = 0, stage_bytes = 0;
   char* ws = nullptr;
   hipEvent_t upload_done = nullptr;
 };
@@ -212,8 +215,8 @@ namespace {
 // CU streams the same number of bytes whatever the spread of sequence
 // lengths.  A workgroup's range becomes one segment per (sequence, group) it
 // touches (cut further so a segment caches at most 511 block ids).  A
-// (sequence, group) with several segments writes partials; the workgroup
-// drawing its last ticket merges them in the same launch.  HW: the largest
+// (sequence, group) with several segments writes partials, which a second
+// small launch merges.  HW: the largest
 // of 8, 4, 2, 1 that divides Hkv, so the 8 waves read all HW heads of a slot
 // (HW x D x 2 contiguous bytes) together.
 // Units (16 keys x one kv-head group) and workgroups of a page-balanced plan.
@@ -238,14 +241,13 @@ BalancedShape balanced_shape(const gllm_attn_plan* p, int cus, int heads_req) {
   return b;
 }
 
-// Page-balanced plans pay a partial write, an L2 write-back (agent-scope
-// release) and a ticket per segment, and the merges of the last segments
-// sit on the launch's tail: measured on MI355X this wins when a workgroup
-// streams enough keys and loses to the split planner below that.  D=64:
-// from ~2048 keys (128 units) per workgroup.  D=128 (Hkv 8, one workgroup per
-// CU): the split planner is 3-3.5% faster at 128-137 units per workgroup, the
-// two are within 1% from 248 to 514, and page-balanced is 0.6-5% faster at
-// 740-770; the cut sits between the measured points.
+// Keys (16-key units) per workgroup from which a decode-only batch is
+// page-balanced whatever its spread of lengths.  Below it, plans of a few items
+// per CU even out by themselves and save the partials and their merge (256
+// sequences of 256-4096 keys, 140 units: 388 us against 402); see also
+// the uneven-load rule in gllm_attn_plan_create.  D=128 (Hkv 8, one workgroup
+// per CU): page-balanced is 0.6-5% faster at 740-770 units, the two within 1%
+// from 248 to 514.
 int64_t balanced_min_units_per_wg(int D) { return D == 128 ? 192 : 128; }
 
 // wgs > 0: that many workgroups (a mixed launch's decode share), else one
@@ -265,6 +267,8 @@ void plan_balanced_decode(gllm_attn_plan* p, int cus, int heads_req, int64_t wgs
   p->split_len = 0;
   p->n_decode_seqs = 0;
   p->segs.clear();
+  p->head_groups = hgroups;
+  p->merge.assign((size_t)p->num_seqs * hgroups, MergeInfo{0, 0});
   p->seg_ptr.assign((size_t)W + 1, 0);
   std::vector<int32_t> seg_wg;
   int64_t u0 = 0, j = 0;
@@ -285,7 +289,6 @@ void plan_balanced_decode(gllm_attn_plan* p, int cus, int heads_req, int64_t wgs
         sg.k0 = (int32_t)(16 * u);
         sg.k1 = (int32_t)std::min<int64_t>(L, 16 * (u + take));
         sg.q_row_start = si.q_row_start; sg.ctx_len = si.ctx_len; sg.q_len = si.q_len;
-        sg.ticket = i * hgroups + hg;
         p->segs.push_back(sg);
         seg_wg.push_back((int32_t)j);
         u += take;
@@ -294,6 +297,7 @@ void plan_balanced_decode(gllm_attn_plan* p, int cus, int heads_req, int64_t wgs
       const int nseg = (int)(p->segs.size() - first);
       const int32_t pbase = (int32_t)p->n_partials;
       if (nseg > 1) p->n_partials += (int64_t)hw * nseg;
+      p->merge[(size_t)i * hgroups + hg] = MergeInfo{pbase, nseg};
       for (int k = 0; k < nseg; ++k) {
         DecodeSeg& sg = p->segs[first + k];
         sg.nseg = nseg; sg.ord = k; sg.pbase = nseg > 1 ? pbase : 0;
@@ -633,7 +637,7 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
   p->num_seqs = num_seqs; p->Hq = num_q_heads; p->Hkv = num_kv_heads; p->D = head_dim;
   p->bs = block_size; p->dtype = dtype; p->mfma = mfma;
   p->seqs.resize(num_seqs);
-  int64_t row = 0, decode_tokens = 0, tile_wgs = 0;
+  int64_t row = 0, tile_wgs = 0;
   for (int i = 0; i < num_seqs; ++i) {
     const int32_t ql = query_lens[i], sl = seq_lens[i];
     if (ql < 1 || sl < ql) {
@@ -653,7 +657,6 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     p->max_q = std::max(p->max_q, ql);
     if (ql < kTileMinRows) p->max_stream_q = std::max(p->max_stream_q, ql);
     else tile_wgs += ((int64_t)ql * G + kTileCols - 1) / kTileCols * num_kv_heads;
-    if (mfma && ql * G <= 16) decode_tokens += sl;
   }
   p->total_rows = q_seq_stride > 0 ? (int64_t)num_seqs * q_seq_stride : row;
   if (p->total_rows > INT32_MAX) {
@@ -731,13 +734,31 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
       if (fills) {
         best_S = cap;
       } else {
-        // about half as many items as resident slots, at least 256 keys each:
-        // a split's partial write and merge cost more than the parallelism
-        // of smaller ones buys (measured: 2 x 8000-key 8B sequences 48.8 ->
-        // 38.7 us, config (a)'s 16-layer bf16 decode step 229 -> 194 us)
+        // the shortest splits (of at least 128 keys) whose items still get a CU
+        // each: a CU streams ~30 GB/s whether it holds one item or two, so one
+        // item more than CUs costs a whole item's time (4 sequences of 3000-7000
+        // keys, 8B heads: 208 items 21.4 us, 308 items 30.0, 132 items 25.7),
+        // and shorter ones pay more start-up than they save.  In a mixed launch,
+        // whose prefill items take CUs too, about half as many items as slots.
         const int64_t hg = (num_kv_heads + best_hw - 1) / best_hw;
-        best_S = (2 * decode_tokens * hg + target - 1) / std::max<int64_t>(target, 1);
-        best_S = std::max<int64_t>((best_S + 31) / 32 * 32, 256);
+        int64_t decode_tokens = 0;
+        for (const SeqInfo& s : p->seqs)
+          if (s.q_len * G <= 16) decode_tokens += s.ctx_len + s.q_len;
+        const auto items = [&](int64_t S) {
+          int64_t n = 0;
+          for (const SeqInfo& s : p->seqs)
+            if (s.q_len * G <= 16) n += ((s.ctx_len + s.q_len + S - 1) / S) * hg;
+          return n;
+        };
+        int64_t lo = 4, hi = cap / 32;     // in 32-key units; items(S) falls as S grows
+        while (lo < hi) {
+          const int64_t mid = (lo + hi) / 2;
+          if (items(32 * mid) <= cus) hi = mid;
+          else lo = mid + 1;
+        }
+        best_S = 32 * lo;
+        if (n_pf > 0)
+          best_S = std::max<int64_t>(((2 * decode_tokens * hg + target - 1) / target + 31) / 32 * 32, 256);
       }
     }
     best_S = std::min(best_S, cap);
@@ -751,6 +772,8 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     const int hgroups = (num_kv_heads + best_hw - 1) / best_hw;
     const int64_t S = best_S;
     p->split_len = (int32_t)S;
+    p->head_groups = hgroups;
+    p->merge.assign((size_t)num_seqs * hgroups, MergeInfo{0, 0});
     struct Keyed { int64_t work; WorkItem it; };
     std::vector<Keyed> pf, dc;
     for (int i = 0; i < num_seqs; ++i) {
@@ -766,7 +789,9 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
         s.nsplits = (int32_t)((L + len - 1) / len);
         len = split_len_of(L, s.nsplits);
         s.partial_base = (int32_t)p->n_partials;
-        if (s.nsplits > 1) p->n_partials += (int64_t)num_kv_heads * s.nsplits;
+        if (s.nsplits > 1) p->n_partials += (int64_t)hgroups * best_hw * s.nsplits;
+        for (int hg = 0; hg < hgroups; ++hg)
+          p->merge[(size_t)i * hgroups + hg] = MergeInfo{s.partial_base + hg * best_hw * s.nsplits, s.nsplits};
         for (int sp = 0; sp < s.nsplits; ++sp)
           for (int hg = 0; hg < hgroups; ++hg) {
             const int64_t keys = std::min<int64_t>(L, (int64_t)(sp + 1) * len) - (int64_t)sp * len;
@@ -783,6 +808,31 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     // Longest work first so the tail is made of short items.
     std::stable_sort(pf.begin(), pf.end(), [](const Keyed& x, const Keyed& y) { return x.work > y.work; });
     std::stable_sort(dc.begin(), dc.end(), [](const Keyed& x, const Keyed& y) { return x.work > y.work; });
+    // A decode-only batch of fewer than two items per CU whose items leave the
+    // CUs unevenly loaded goes page-balanced: its partials and their merge cost
+    // ~8 us, which a CU streams 256 KB in.  Measured (split / page-balanced us,
+    // 8B heads; longest CU's excess over the mean): 48 sequences of 1100 keys
+    // 57.4 / 50.3 (excess 275 KB), 32 of 500-3000 65.6 / 49.7 (660 KB), 40 of
+    // 4000 161 / 121 (1.5 MB); 90 of 500-2000 92.3 / 94.5 (190 KB), 160 of
+    // 300-900 84.1 / 85.7 (210 KB).
+    if (pf.empty() && split_tokens == 0 && !decode_heads_per_wg && dc.size() < 2 * (size_t)cus) {
+      std::vector<int64_t> load((size_t)cus, 0);   // min-heap of the CUs' keys, longest item first
+      int64_t total = 0, longest = 0;
+      for (const Keyed& k : dc) {
+        std::pop_heap(load.begin(), load.end(), std::greater<int64_t>());
+        load.back() += k.work;
+        total += k.work;
+        longest = std::max(longest, load.back());
+        std::push_heap(load.begin(), load.end(), std::greater<int64_t>());
+      }
+      const int64_t key_bytes = (int64_t)best_hw * head_dim * 4;   // K and V, 16-bit
+      if ((longest - total / cus) * key_bytes > (int64_t(256) << 10)) {
+        p->n_partials = 0;
+        balanced = true;
+        plan_balanced_decode(p, cus, 0, 0);
+      }
+    }
+    if (!balanced) {
     // Workgroups are dispatched slot-major: while every slot is free, item k
     // and item k + cus land on the same CU, and the older (first) one wins
     // the CU's memory pipeline.
@@ -839,6 +889,7 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
       return fail(GLLM_ATTN_EINVAL, "too many work items");
     }
     }
+    }
   }
   if (!mfma && p->tile_min_q > 0) {
     // Generic plan: one item per kTileCols (query row, head) columns of a kv
@@ -868,18 +919,20 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     return fail(GLLM_ATTN_EINVAL, "too many split partials");
   }
 
-  // Workspace layout: items | seqs | segments | segment ranges | tickets |
+  // Workspace layout: items | seqs | segments | segment ranges | merge table |
   // partial (m, l) | partial acc.
+  if (p->n_partials == 0) p->merge.clear();
   size_t o = 0;
   p->off_items = o; o = align256(o + p->items.size() * sizeof(WorkItem));
   p->off_seqs = o; o = align256(o + p->seqs.size() * sizeof(SeqInfo));
   p->off_segs = o; o = align256(o + p->segs.size() * sizeof(DecodeSeg));
   p->off_segptr = o; o = align256(o + p->seg_ptr.size() * sizeof(int32_t));
-  p->off_ctr = o; o = align256(o + (size_t)num_seqs * num_kv_heads * sizeof(int32_t));
+  p->off_merge = o; o = align256(o + p->merge.size() * sizeof(MergeInfo));
+  const size_t stage = o;                        // uploaded part
+  p->stage_bytes = stage;
   p->off_ml = o; o = align256(o + (size_t)p->n_partials * 16 * 2 * sizeof(float));
   p->off_part = o; o = align256(o + (size_t)p->n_partials * 16 * head_dim * sizeof(float));
   p->ws_bytes = std::max<size_t>(o, 256);
-  const size_t stage = p->off_ctr;
   if (stage > 0) {
     p->pinned = pinned_pool().acquire(stage, &p->pinned_cap);
     if (!p->pinned) {
@@ -896,6 +949,8 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     if (!p->segs.empty()) std::memcpy((char*)p->pinned + p->off_segs, p->segs.data(), p->segs.size() * sizeof(DecodeSeg));
     if (!p->seg_ptr.empty())
       std::memcpy((char*)p->pinned + p->off_segptr, p->seg_ptr.data(), p->seg_ptr.size() * sizeof(int32_t));
+    if (!p->merge.empty())
+      std::memcpy((char*)p->pinned + p->off_merge, p->merge.data(), p->merge.size() * sizeof(MergeInfo));
   }
   *out = p;
   return ok();
@@ -921,12 +976,11 @@ int gllm_attn_plan_upload(gllm_attn_plan* p, void* workspace, size_t bytes, void
   if (((uintptr_t)workspace & 255) != 0) return fail(GLLM_ATTN_EINVAL, "workspace must be 256-byte aligned");
   hipStream_t st = (hipStream_t)stream;
   p->ws = (char*)workspace;
-  if (p->off_ctr > 0) {
-    hipError_t e = hipMemcpyAsync(p->ws, p->pinned, p->off_ctr, hipMemcpyHostToDevice, st);
+  hipError_t e = hipSuccess;
+  if (p->stage_bytes > 0) {
+    e = hipMemcpyAsync(p->ws, p->pinned, p->stage_bytes, hipMemcpyHostToDevice, st);
     if (e != hipSuccess) return hip_check(e, "plan upload copy");
   }
-  hipError_t e = launch_fill_zero_i32((int32_t*)(p->ws + p->off_ctr), (int64_t)p->num_seqs * p->Hkv, st);
-  if (e != hipSuccess) return hip_check(e, "ticket clear");
   if (!p->upload_done) {
     e = hipEventCreateWithFlags(&p->upload_done, hipEventDisableTiming);
     if (e != hipSuccess) return hip_check(e, "hipEventCreate");
@@ -1000,7 +1054,8 @@ static int paged_attention_impl(const gllm_attn_plan* p, const void* q, int64_t 
     a.n_items = a.n_seg_wgs + (int32_t)p->items.size();   // decode workgroups, then any prefill items
   }
   a.num_seqs = p->num_seqs;
-  a.counters = (int32_t*)(p->ws + p->off_ctr);
+  a.merge = (const MergeInfo*)(p->ws + p->off_merge);
+  a.head_groups = p->head_groups;
   a.partial_ml = (float*)(p->ws + p->off_ml);
   a.partials = (float*)(p->ws + p->off_part);
   a.split_len = p->split_len;

@@ -351,8 +351,8 @@ struct WorkItem {
 // Key range [k0, k1) of one (sequence, kv-head group) for the page-balanced
 // decode launch: the workgroups split the batch's 16-key units evenly, so a
 // sequence's keys may be spread over several workgroups.  Its nseg segments
-// write partials at pbase + head_in_group * nseg + ord; the workgroup that
-// draws the last ticket of counters[ticket] merges them.
+// write partials at pbase + head_in_group * nseg + ord, which
+// merge_splits_kernel combines.
 struct DecodeSeg {
   int32_t seq;
   int32_t hg;            // kv-head group (heads hg * HW .. hg * HW + HW - 1)
@@ -363,8 +363,12 @@ struct DecodeSeg {
   int32_t nseg;          // segments of this (sequence, group); 1 = written directly
   int32_t pbase;
   int32_t ord;
-  int32_t ticket;        // counter index of this (sequence, group)
-  int32_t pad;
+};
+
+// Partials of one (sequence, kv-head group): head i of the group has `count`
+// of them from pbase + i * count on (count <= 1: none, the task wrote the output).
+struct MergeInfo {
+  int32_t pbase, count;
 };
 
 }  // namespace gllm

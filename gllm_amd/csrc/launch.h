@@ -91,7 +91,8 @@ struct AttnArgs {
   int64_t n_partials;
   float* partials;            // [n_partials][16][D] fp32
   float* partial_ml;          // [n_partials][16][2] fp32 (running max in log2 units, sum)
-  int32_t* counters;          // [num_seqs * Hkv] split tickets, zero between launches
+  const MergeInfo* merge;     // [num_seqs * head_groups] partials of each (sequence, kv-head group)
+  int32_t head_groups;
   // page-balanced decode (n_segs > 0): workgroup w runs segs[seg_ptr[w] .. seg_ptr[w + 1])
   const DecodeSeg* segs;
   const int32_t* seg_ptr;
@@ -182,6 +183,5 @@ hipError_t launch_dense_attention_mfma(const AttnArgs& a, int B, int Tq, hipStre
 // Generic kernels: max_q the largest query length, max_stream_q the largest of
 // the sequences on the stream kernel (0: every sequence is tiled)
 hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, hipStream_t stream);
-hipError_t launch_fill_zero_i32(int32_t* p, int64_t n, hipStream_t stream);
 
 }  // namespace gllm

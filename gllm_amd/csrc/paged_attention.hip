@@ -13,9 +13,9 @@
 //   HBM straight into MFMA operand registers (16-byte loads) through a
 //   prefetch ring; online softmax in fp32 (log2 domain, lazy rescale);
 //   O^T += V^T P^T on v_mfma_f32_16x16x16_bf16 with V transposed through LDS
-//   by ds_read_b64_tr_b16.  Split plans merge split partials in a second
-//   small launch; page-balanced plans deal equal key ranges to the
-//   workgroups and merge in the same launch (split tickets).
+//   by ds_read_b64_tr_b16.  Split plans cut long sequences into equal key
+//   ranges, page-balanced plans deal equal key ranges to the workgroups; a
+//   second small launch merges the partials of both.
 // Prefill (one 8-wave workgroup per (sequence, kv head, 8 row tiles of 32)):
 //   K/V tiles of 64 keys staged in LDS, S^T = K Q^T and O^T += V^T P^T on
 //   v_mfma_f32_32x32x16_bf16, flash-style running max/sum, causal tile skip.
@@ -84,10 +84,9 @@ __device__ __forceinline__ u32x4 chunk_elems(const u32x4* raw, int kk) {
 // One decode task: keys [kbeg, kend) of one sequence for HW kv heads.
 struct DecodeTask {
   int seq, hg, kbeg, kend, q_row_start, ctx_len, q_len;
-  int nseg;     // tasks of this (sequence, head group); 1: normalise and write the output
+  int nseg;     // tasks of this (sequence, head group); 1: normalise and write the output, else a partial for merge_splits_kernel
   int pbase;    // partial of head i of the group: pbase + i * nseg + ord
   int ord;
-  int ticket;   // >= 0: counter whose last ticket merges the partials here; < 0: merge_splits does
 };
 
 // New tokens written by the attention launch (a.k_new != null): the task whose
@@ -144,7 +143,7 @@ __device__ __forceinline__ void write_new_keys(const AttnArgs& a, const DecodeTa
 // Runs one task with every wave of the workgroup; returns with the workgroup
 // converged (no early exit), so a workgroup can run several tasks in a row.
 template <typename T, int D, int HW, int KW, bool KV8>
-__device__ __forceinline__ void decode_task(const AttnArgs& a, const DecodeTask& tk, char* lds, int* ticket_lds) {
+__device__ __forceinline__ void decode_task(const AttnArgs& a, const DecodeTask& tk, char* lds) {
   constexpr int NW = HW * KW;
   constexpr int E = KV8 ? 1 : 2;   // bytes per cached element
   using Cfg = DecodeCfg<D, NW>;
@@ -420,83 +419,6 @@ __device__ __forceinline__ void decode_task(const AttnArgs& a, const DecodeTask&
       a.partial_ml[((pfirst + tk.ord) * 16 + n) * 2 + 1] = lt;
     }
   }
-  if (tk.ticket < 0) return;
-  // Ticket: the workgroup that completes a (sequence, group) last merges its
-  // partials.  The barrier orders every wave's partial stores before thread
-  // 0's agent-scope release (L2 write-back, so workgroups on other XCDs see
-  // them); the last ticket holder acquires (L2 invalidate) before reading.
-  // Nobody waits on anybody: a workgroup that is not last simply moves on.
-  __syncthreads();
-  if (tid == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    const int t = __hip_atomic_fetch_add(a.counters + tk.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (t == tk.nseg - 1) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      // every ticket of this launch is drawn: re-arm the counter for the next one
-      __hip_atomic_store(a.counters + tk.ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    *ticket_lds = t;
-  }
-  __syncthreads();
-  const bool last = *ticket_lds == tk.nseg - 1;
-  if (!last || !lead || !head_ok) return;
-  // LSE merge, latency-bound (it is the launch's tail): the 16 row lanes of
-  // each 16-lane group are (row mr, partial slot ps) pairs, R rows x PS
-  // slots, and slot ps takes partials ps, ps + PS, ..., CH of them per
-  // round trip with all their loads in flight; the slots are then combined
-  // through shuffles in slot order.  The sums depend only on the partials,
-  // not on which workgroup merges.
-  constexpr int CH = 2;
-  const int PS = 16 / R;
-  const int mr = n % R, ps = n / R;
-  const bool mact = ps < PS;
-  float Mx = kNegInf, Lx = 0.f;
-  f32x4 ox[ND];
-#pragma unroll
-  for (int d = 0; d < ND; ++d) ox[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto combine = [&](float m2, float l2, const f32x4 (&o2)[ND]) {
-    const float nM = fmaxf(Mx, m2);
-    if (nM == kNegInf) return;
-    const float w1 = fast_exp2(Mx - nM), w2 = fast_exp2(m2 - nM);
-    Lx = Lx * w1 + l2 * w2;
-#pragma unroll
-    for (int d = 0; d < ND; ++d) ox[d] = ox[d] * w1 + o2[d] * w2;
-    Mx = nM;
-  };
-  for (int o0 = 0; o0 < tk.nseg; o0 += PS * CH) {
-    float mm[CH], ll[CH];
-    f32x4 vv[CH][ND];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int o = o0 + c * PS + ps;
-      const bool v = mact && o < tk.nseg;
-      const int64_t pi = (pfirst + (v ? o : 0)) * 16 + mr;
-      mm[c] = v ? a.partial_ml[pi * 2] : kNegInf;
-      ll[c] = v ? a.partial_ml[pi * 2 + 1] : 0.f;
-      const float* pa = a.partials + pi * D + 4 * grp;
-#pragma unroll
-      for (int d = 0; d < ND; ++d) vv[c][d] = v ? *reinterpret_cast<const f32x4*>(pa + 16 * d) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int c = 0; c < CH; ++c) combine(mm[c], ll[c], vv[c]);
-  }
-  // slot k's state moves to slot 0 (lanes mr + R k -> mr, same 16-dim group)
-  for (int k = 1; k < PS; ++k) {
-    const int src = (lane & 48) | min(15, mr + R * k);
-    const float m2 = __shfl(Mx, src, 64), l2 = __shfl(Lx, src, 64);
-    f32x4 o2[ND];
-#pragma unroll
-    for (int d = 0; d < ND; ++d)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) o2[d][j] = __shfl(ox[d][j], src, 64);
-    if (ps == 0) combine(m2, l2, o2);
-  }
-  if (!row_ok) return;   // ps == 0 lanes: mr == n
-  const float inv = 1.f / Lx;
-  T* op = (T*)a.out + qrow * a.out_row_stride + (int64_t)qh * D + 4 * grp;
-#pragma unroll
-  for (int d = 0; d < ND; ++d)
-    st8(op + 16 * d, u32x2{E16<T>::pack2(ox[d][0] * inv, ox[d][1] * inv), E16<T>::pack2(ox[d][2] * inv, ox[d][3] * inv)});
 }
 
 // One decode work item of the split-launch planner (split it.a of the
@@ -517,39 +439,82 @@ __device__ __forceinline__ void decode_wg(const AttnArgs& a, const WorkItem& it,
   tk.nseg = it.nsplits;
   tk.pbase = it.partial_base + tk.hg * HW * it.nsplits;
   tk.ord = it.a;
-  tk.ticket = -1;
-  decode_task<T, D, HW, KW, KV8>(a, tk, lds, nullptr);
+  decode_task<T, D, HW, KW, KV8>(a, tk, lds);
 }
 
 // Combines the split partials of every (sequence, kv head) whose sequence
-// was split: one wave per (sequence, kv head); softmax-weighted (LSE) merge.
+// was split (softmax-weighted LSE merge).  Latency-bound: one 8-wave workgroup
+// per (sequence, kv head); a thread takes 4 dims of a row and every NG-th
+// split, CH splits' loads in flight at a time, and the NG groups meet in LDS
+// (a wave that walked the splits one after another took 15.4 us for 4
+// sequences of 5000 keys in 9 splits each, this 4.5).
+constexpr int kMergeThreads = 512;
 template <typename T, int D>
-__global__ void __launch_bounds__(64) merge_splits_kernel(AttnArgs a) {
-  const int seq = blockIdx.x / a.num_kv_heads, kvh = blockIdx.x - seq * a.num_kv_heads;
-  const SeqInfo si = a.seqs[seq];
-  if (si.nsplits <= 1) return;
-  const int G = a.num_q_heads / a.num_kv_heads;
-  const int R = si.q_len * G;
+__global__ void __launch_bounds__(kMergeThreads) merge_splits_kernel(AttnArgs a) {
+  constexpr int CH = 8;
   constexpr int CPR = D / 4;
-  const int64_t pbase = (int64_t)si.partial_base + (int64_t)kvh * si.nsplits;
-  for (int e = threadIdx.x; e < R * CPR; e += 64) {
-    const int row = e / CPR, d4 = (e - row * CPR) * 4;
-    float M = kNegInf;
-    for (int sp = 0; sp < si.nsplits; ++sp) M = fmaxf(M, a.partial_ml[((pbase + sp) * 16 + row) * 2]);
-    const float Mu = M == kNegInf ? 0.f : M;
-    float Ls = 0.f;
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int sp = 0; sp < si.nsplits; ++sp) {
-      const float* ml = a.partial_ml + ((pbase + sp) * 16 + row) * 2;
-      const float w = fast_exp2(ml[0] - Mu);
-      Ls += w * ml[1];
-      o += w * *reinterpret_cast<const f32x4*>(a.partials + ((pbase + sp) * 16 + row) * D + d4);
+  static_assert(16 * CPR <= kMergeThreads, "a thread per 4 dims of 16 rows");
+  __shared__ __attribute__((aligned(16))) f32x4 so[kMergeThreads];
+  __shared__ float sm[kMergeThreads], sl[kMergeThreads];
+  const int seq = blockIdx.x / a.num_kv_heads, kvh = blockIdx.x - seq * a.num_kv_heads;
+  const int hg = kvh / a.heads_per_wg;
+  const MergeInfo mi = a.merge[seq * a.head_groups + hg];
+  const int ns = mi.count;
+  if (ns <= 1) return;
+  const SeqInfo si = a.seqs[seq];
+  const int G = a.num_q_heads / a.num_kv_heads;
+  const int E = si.q_len * G * CPR;             // elements: (row, 4 dims); at most 16 rows
+  const int NG = ns <= CH ? 1 : kMergeThreads / E;
+  const int grp = threadIdx.x / E, e = threadIdx.x - grp * E;
+  if (NG == 1 && grp > 0) return;               // one round trip for one group: nothing to meet
+  const int row = e / CPR, d4 = (e - row * CPR) * 4;
+  const int64_t pbase = (int64_t)mi.pbase + (int64_t)(kvh - hg * a.heads_per_wg) * ns;
+  const float* ml = a.partial_ml + (pbase * 16 + row) * 2;
+  const float* pa = a.partials + (pbase * 16 + row) * D + d4;
+  float M = kNegInf, Ls = 0.f;
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  auto add = [&](float m, float l, f32x4 v) {
+    Ls += m * l;
+    o += m * v;
+  };
+  for (int s0 = grp; grp < NG && s0 < ns; s0 += NG * CH) {
+    u32x2 x[CH];
+    f32x4 v[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {              // splits past the last one re-read it, with weight 0
+      const int64_t sp = min(s0 + NG * c, ns - 1);
+      x[c] = *reinterpret_cast<const u32x2*>(ml + sp * 32);
+      v[c] = *reinterpret_cast<const f32x4*>(pa + sp * 16 * D);
     }
-    const float inv = 1.f / Ls;
-    const int rr = row / G, gg = row - rr * G;
-    T* op = (T*)a.out + (si.q_row_start + rr) * a.out_row_stride + (int64_t)(kvh * G + gg) * D + d4;
-    st8(op, u32x2{E16<T>::pack2(o[0] * inv, o[1] * inv), E16<T>::pack2(o[2] * inv, o[3] * inv)});
+    float Mn = M;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) Mn = fmaxf(Mn, __uint_as_float(x[c][0]));
+    const float Mu = Mn == kNegInf ? 0.f : Mn;
+    const float al = fast_exp2(M - Mu);
+    Ls *= al;
+    o *= al;
+#pragma unroll
+    for (int c = 0; c < CH; ++c)                // fixed order: deterministic sums
+      if (s0 + NG * c < ns) add(fast_exp2(__uint_as_float(x[c][0]) - Mu), __uint_as_float(x[c][1]), v[c]);
+    M = Mn;
   }
+  if (NG > 1) {
+    so[threadIdx.x] = o;
+    sm[threadIdx.x] = M;
+    sl[threadIdx.x] = Ls;
+    __syncthreads();
+    if (grp != 0) return;
+    float Mt = kNegInf;
+    for (int k = 0; k < NG; ++k) Mt = fmaxf(Mt, sm[k * E + e]);
+    const float Mu = Mt == kNegInf ? 0.f : Mt;
+    Ls = 0.f;
+    o = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < NG; ++k) add(fast_exp2(sm[k * E + e] - Mu), sl[k * E + e], so[k * E + e]);
+  }
+  const float inv = 1.f / Ls;
+  const int rr = row / G, gg = row - rr * G;
+  T* op = (T*)a.out + (si.q_row_start + rr) * a.out_row_stride + (int64_t)(kvh * G + gg) * D + d4;
+  st8(op, u32x2{E16<T>::pack2(o[0] * inv, o[1] * inv), E16<T>::pack2(o[2] * inv, o[3] * inv)});
 }
 
 // ============================================================== prefill
@@ -1257,14 +1222,13 @@ template <typename T, int D, int HW, int KW, bool KV8>
 __global__ void __launch_bounds__(64 * HW * KW) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 decode_balanced_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[DecodeCfg<D, HW * KW>::kLdsBytes];
-  __shared__ int ticket;
   const int s0 = a.seg_ptr[blockIdx.x], s1 = a.seg_ptr[blockIdx.x + 1];
   for (int s = s0; s < s1; ++s) {
     if (s > s0) __syncthreads();
     const DecodeSeg sg = a.segs[s];
     const DecodeTask tk{sg.seq, sg.hg, sg.k0, sg.k1, sg.q_row_start, sg.ctx_len, sg.q_len,
-                        sg.nseg, sg.pbase, sg.ord, sg.ticket};
-    decode_task<T, D, HW, KW, KV8>(a, tk, lds, &ticket);
+                        sg.nseg, sg.pbase, sg.ord};
+    decode_task<T, D, HW, KW, KV8>(a, tk, lds);
   }
 }
 
@@ -1275,7 +1239,6 @@ decode_balanced_kernel(AttnArgs a) {
 template <typename T, int D, int HW, bool KV8>
 __global__ void __launch_bounds__(64 * kWaves) mixed_balanced_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[MixedLds<D, true, true, kWaves>::kBytes];
-  __shared__ int ticket;
   const int b = blockIdx.x;
   if (b >= a.n_seg_wgs) {
     const WorkItem it = a.items[b - a.n_seg_wgs];
@@ -1287,8 +1250,8 @@ __global__ void __launch_bounds__(64 * kWaves) mixed_balanced_kernel(AttnArgs a)
     if (s > s0) __syncthreads();
     const DecodeSeg sg = a.segs[s];
     const DecodeTask tk{sg.seq, sg.hg, sg.k0, sg.k1, sg.q_row_start, sg.ctx_len, sg.q_len,
-                        sg.nseg, sg.pbase, sg.ord, sg.ticket};
-    decode_task<T, D, HW, kWaves / HW, KV8>(a, tk, lds, &ticket);
+                        sg.nseg, sg.pbase, sg.ord};
+    decode_task<T, D, HW, kWaves / HW, KV8>(a, tk, lds);
   }
 }
 
@@ -1355,15 +1318,14 @@ static hipError_t launch_mixed_balanced(const AttnArgs& a, hipStream_t st) {
 template <typename T, int D, bool KV8>
 static hipError_t launch_paged_d(const AttnArgs& a, bool pf, bool dc, hipStream_t st) {
   const int hw = a.heads_per_wg, nw = a.decode_waves;
+  hipError_t e;
   if (a.n_segs > 0) {
     if (nw != kWaves || (pf && a.prefill_waves != kWaves) || a.n_seg_wgs <= 0 || a.n_seg_wgs > a.n_items)
       return hipErrorInvalidValue;
-    if (pf) return dc ? launch_mixed_balanced<T, D, KV8>(a, st) : hipErrorInvalidValue;
-    return launch_decode_balanced<T, D, KV8>(a, st);
-  }
-  if (pf && (a.prefill_waves != (dc ? kWaves : kPrefillOnlyWaves) || (dc && nw != kWaves)))
-    return hipErrorInvalidValue;
-  if (nw == 8) {
+    if (pf && !dc) return hipErrorInvalidValue;
+    e = pf ? launch_mixed_balanced<T, D, KV8>(a, st) : launch_decode_balanced<T, D, KV8>(a, st);
+  } else {
+    if (nw != kWaves || (pf && a.prefill_waves != (dc ? kWaves : kPrefillOnlyWaves))) return hipErrorInvalidValue;
     switch (hw) {
       case 1: launch_paged_hk<T, D, 1, 8, KV8>(a, pf, dc, st); break;
       case 2: launch_paged_hk<T, D, 2, 4, KV8>(a, pf, dc, st); break;
@@ -1371,12 +1333,10 @@ static hipError_t launch_paged_d(const AttnArgs& a, bool pf, bool dc, hipStream_
       case 8: launch_paged_hk<T, D, 8, 1, KV8>(a, pf, dc, st); break;
       default: return hipErrorInvalidValue;
     }
-  } else {
-    return hipErrorInvalidValue;
+    e = hipGetLastError();
   }
-  hipError_t e = hipGetLastError();
   if (e != hipSuccess || !dc || a.n_partials == 0) return e;
-  hipLaunchKernelGGL((merge_splits_kernel<T, D>), dim3(a.num_seqs * a.num_kv_heads), dim3(64), 0, st, a);
+  hipLaunchKernelGGL((merge_splits_kernel<T, D>), dim3(a.num_seqs * a.num_kv_heads), dim3(kMergeThreads), 0, st, a);
   return hipGetLastError();
 }
 
@@ -1435,17 +1395,6 @@ hipError_t launch_dense_attention_mfma(const AttnArgs& a, int B, int Tq, hipStre
   return hipErrorInvalidValue;
 }
 
-__global__ void fill_zero_i32_kernel(int32_t* p, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = 0;
-}
-
-hipError_t launch_fill_zero_i32(int32_t* p, int64_t n, hipStream_t st) {
-  if (n <= 0) return hipSuccess;
-  int64_t blocks = (n + 255) / 256;
-  if (blocks > 1024) blocks = 1024;
-  hipLaunchKernelGGL(fill_zero_i32_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p, n);
-  return hipGetLastError();
-}
 #endif  // GLLM_PAGED_F16
 
 }  // namespace gllm

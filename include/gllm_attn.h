@@ -199,9 +199,10 @@ int gllm_rope_kv_write(const void* q, void* q_out, const void* k, const void* v,
  * the batch and the CU count.  split_tokens == GLLM_SPLIT_BALANCED (-1) plans
  * the decode sequences page-balanced: their keys (16-key units per sequence
  * and kv-head group) are dealt out evenly to one workgroup per resident CU
- * slot, and sequences spread over several workgroups are merged inside the
- * same launch (split tickets); 0 picks it for decode-only batches whose
- * workgroups would each stream >= 2048 keys.  In a mixed batch (only on
+ * slot, and sequences spread over several workgroups are merged by a second
+ * small launch; 0 picks it for decode-only batches whose workgroups would each
+ * stream >= 2048 keys, and for those whose unsplit items would load the CUs
+ * unevenly.  In a mixed batch (only on
  * request) the decode share goes to a multiple of 8 workgroups sized by a
  * cost model, and one workgroup per prefill item follows them on the other
  * CUs.  No device work happens here.
@@ -211,7 +212,7 @@ int gllm_attn_plan_create(gllm_attn_plan** plan, const int32_t* query_lens,
                           int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
                           int32_t block_size, int32_t dtype, int32_t split_tokens,
                           int32_t decode_heads_per_wg);
-/* Device bytes the plan needs (work list, split partials, tickets). */
+/* Device bytes the plan needs (work list, split partials). */
 size_t gllm_attn_plan_workspace_bytes(const gllm_attn_plan* plan);
 /* Stream-ordered upload of the plan into `workspace` (>= workspace_bytes).
  * The workspace must stay alive and untouched while launches use the plan. */

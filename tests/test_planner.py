@@ -1,0 +1,50 @@
+"""The decode planner's choices (host code, no GPU): how a small batch is split
+and when an uneven one goes page-balanced."""
+import ctypes
+
+import pytest
+
+from gllm_amd import _lib
+
+CUS = 256      # what the planner assumes without a device
+
+
+def _info(q, L, Hq=32, Hkv=8, D=128, split=0, hw=0):
+    lib = _lib.load()
+    h = ctypes.c_void_p()
+    arr = lambda v: (ctypes.c_int32 * len(v))(*v)
+    _lib.check(lib.gllm_attn_plan_create(ctypes.byref(h), arr(q), arr(L), len(L), 0, Hq, Hkv, D, 16,
+                                         _lib.DTYPE_BF16, split, hw))
+    out = (ctypes.c_int64 * 10)()
+    _lib.check(lib.gllm_attn_plan_info(h, out, 10))
+    nbytes = lib.gllm_attn_plan_workspace_bytes(h)
+    lib.gllm_attn_plan_destroy(h)
+    keys = ("items", "split", "dec", "pre", "partials", "rows", "hw", "dw", "pw", "segs")
+    return dict(zip(keys, out)), nbytes
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("L", [[1], [127], [300], [2048], [40000], [5000, 3000, 7000, 4200], [500] * 16, [3000] * 16])
+def test_small_batches_get_one_item_per_cu(L, D):
+    i, nbytes = _info([1] * len(L), L, D=D)
+    assert i["segs"] == 0 and i["dec"] == len(L)
+    assert i["items"] <= CUS
+    # splits of at least 128 keys, and no coarser than the CUs ask for
+    assert i["split"] >= 128
+    if i["split"] > 128:
+        finer = sum(-(-x // (i["split"] - 32)) for x in L) * -(-8 // i["hw"])
+        assert finer > CUS
+    assert nbytes >= i["partials"] * 16 * (D + 2) * 4
+
+
+def test_uneven_batches_go_page_balanced():
+    import random
+    r = random.Random(0)
+    uneven = [r.randint(500, 3000) for _ in range(32)]
+    assert _info([1] * 32, uneven)[0]["segs"] > 0
+    assert _info([1] * 32, [1500] * 32)[0]["segs"] == 0          # one equal item per CU
+    assert _info([1] * 40, [4000] * 40)[0]["segs"] > 0           # 1.25 rounds of long items
+    assert _info([1] * 32, uneven, split=1024)[0]["segs"] == 0   # a split length was asked for
+    assert _info([1] * 31 + [64], uneven)[0]["segs"] == 0        # mixed batches only on request
+    many = [r.randint(256, 4096) for _ in range(256)]
+    assert _info([1] * 256, many)[0]["segs"] == 0                # four items per CU even out

@@ -97,6 +97,20 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
 QKV_UNFUSED_FROM = 3072
 
 
+def qkv_fused_ok(x: torch.Tensor, w_q: torch.Tensor, w_k: torch.Tensor, w_v: torch.Tensor,
+                 k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
+    """Whether the fused kernels of :func:`qkv_rope_kv_write` take these rows,
+    weights and caches: bf16 rows of a hidden size that is a multiple of 32, 16-byte
+    aligned, a bf16 or fp8 cache, head dim 64 or 128."""
+    hidden = x.shape[-1]
+    if x.dim() != 2 or hidden % 32 or k_cache.shape[2] not in (64, 128):
+        return False
+    if k_cache.dtype not in (torch.bfloat16, torch.float8_e4m3fn) or v_cache.dtype != k_cache.dtype:
+        return False
+    return all(t.dtype == torch.bfloat16 and t.dim() == 2 and t.shape[1] == hidden and t.stride(1) == 1
+               and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w_q, w_k, w_v))
+
+
 def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tensor, w_v: torch.Tensor,
                       cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       slot_mapping: torch.Tensor, *, rotate_q: bool = True, q_out: torch.Tensor | None = None,
@@ -111,7 +125,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     ``query_lens`` / ``slot_mapping`` as in :func:`rope_kv_write`.  Returns q
     ``[N, Hq, D]`` (rotated if ``rotate_q``) or None when ``w_q`` is None.
     ``split_k``: let batches of few tokens split the hidden dimension over
-    more workgroups (a cached device workspace); False forces the tile kernel.
+    more workgroups (a device workspace); False forces the tile kernel.
     ``unfused_from``: from this many tokens the projections run as three
     ``F.linear`` (hipBLASLt) followed by :func:`rope_kv_write`, which is faster
     there; None runs the fused kernel at any size.  Head dims other than 64
@@ -175,7 +189,8 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     lib = _lib.load()
     qrow = q_out.reshape(-1, Hq * D).stride(0) if q_out is not None else 0
     wsb = lib.gllm_qkv_workspace_bytes(n, hidden, max(Hq, 1), Hkv, D, int(w_q is not None)) if split_k else 0
-    ws = _qkv_workspace(x.device, wsb) if wsb else None
+    # per call, from the caching allocator: calls on other streams have their own
+    ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
     _lib.check(lib.gllm_qkv_rope_kv_write(
         xs.data_ptr(), xs.stride(0), n, hidden, _lib.ptr(w_q), w_q.stride(0) if w_q is not None else 0,
         w_k.data_ptr(), w_k.stride(0), w_v.data_ptr(), w_v.stride(0), _lib.ptr(q_out), qrow, int(bool(rotate_q)),
@@ -183,20 +198,6 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
         tps, cs.data_ptr(), sn.data_ptr(), _lib.ptr(rr), cs.stride(0), max(Hq, 1), Hkv, D,
         _lib.dtype_code(x.dtype), _lib.dtype_code(k_cache.dtype), _lib.ptr(ws), wsb, _lib.stream_ptr(x.device)))
     return q_out
-
-
-_QKV_WS: dict = {}
-
-
-def _qkv_workspace(device, nbytes: int) -> torch.Tensor:
-    """Per-device scratch for the split-K projection (grown on demand, kept;
-    fully rewritten by every call, so never cleared)."""
-    key = torch.device(device)
-    ws = _QKV_WS.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=key)
-        _QKV_WS[key] = ws
-    return ws
 
 
 def rope_rotate(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

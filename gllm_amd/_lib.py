@@ -86,20 +86,22 @@ def check(rc: int) -> None:
     raise RuntimeError(msg)
 
 
+_DTYPE_CODES = {torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16, torch.float16: DTYPE_F16,
+                torch.float8_e4m3fn: DTYPE_FP8_E4M3}
+
+
 def dtype_code(dt: torch.dtype) -> int:
-    if dt == torch.bfloat16:
-        return DTYPE_BF16
-    if dt == torch.float32:
-        return DTYPE_F32
-    if dt == torch.float16:
-        return DTYPE_F16
-    if dt == torch.float8_e4m3fn:
-        return DTYPE_FP8_E4M3
-    raise NotImplementedError(f"dtype {dt} is not supported (float32, bfloat16, float16; float8_e4m3fn for the "
-                              "KV cache)")
+    code = _DTYPE_CODES.get(dt)
+    if code is None:
+        raise NotImplementedError(f"dtype {dt} is not supported (float32, bfloat16, float16; float8_e4m3fn for the "
+                                  "KV cache)")
+    return code
 
 
 def stream_ptr(device: torch.device) -> int:
+    """The hipStream_t of torch's current stream on the device."""
+    if device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)    # without the Stream object around it
     return torch.cuda.current_stream(device).cuda_stream
 
 

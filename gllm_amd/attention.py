@@ -139,6 +139,11 @@ class Attention:
         return F.linear(attn.view(B, Tq, -1), self.W_o.to(x.device))
 
     def _plan(self, meta, dtype, device) -> paged.AttentionPlan:
+        """The step's plan: built by the step's first layer, kept on ``meta``."""
+        plan = getattr(meta, "_gllm_plan", None)
+        if plan is not None:
+            self._block_size = plan.block_size
+            return plan
         plan = plan_for(meta, num_q_heads=self.num_q_heads, num_kv_heads=self.num_kv_heads, head_dim=self.head_dim,
                         dtype=dtype, device=device, block_size_hint=self._block_size)
         self._block_size = plan.block_size

@@ -16,6 +16,10 @@ from . import _lib
 def _rows(t: torch.Tensor, heads: int, head_dim: int, name: str) -> int:
     """Row stride (elements) of a [..., heads, head_dim] tensor whose leading
     dims flatten to rows without a copy."""
+    if t.is_contiguous():                  # the common case, without a look at each dim
+        shape, hd = t.shape, heads * head_dim
+        if len(shape) >= 3 and shape[-1] == head_dim and shape[-2] == heads and t.stride()[-3] == hd:
+            return hd
     if t.dim() < 2 or t.shape[-1] != head_dim or t.shape[-2] != heads:
         raise ValueError(f"{name}: expected [..., {heads}, {head_dim}], got {tuple(t.shape)}")
     if t.stride(-1) != 1 or t.stride(-2) != head_dim:
@@ -30,6 +34,26 @@ def _rows(t: torch.Tensor, heads: int, head_dim: int, name: str) -> int:
         expect *= t.shape[d]
     del lead
     return stride
+
+
+def _table(t: torch.Tensor) -> torch.Tensor:
+    """cos / sin as rows."""
+    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+
+
+def _index_rows(t: torch.Tensor) -> torch.Tensor:
+    """Row indices as one contiguous int64 vector."""
+    if t.dim() == 1 and t.dtype == torch.int64 and t.is_contiguous():
+        return t
+    return t.reshape(-1).to(torch.int64).contiguous()
+
+
+def _cache_rows(k_cache: torch.Tensor, v_cache: torch.Tensor, Hkv: int, D: int) -> None:
+    """Checks that the caches are [num_slots, Hkv, D] with contiguous rows."""
+    for t, nm in ((k_cache, "k_cache"), (v_cache, "v_cache")):
+        shape = t.shape
+        if len(shape) != 3 or shape[1] != Hkv or shape[2] != D or t.stride()[1:] != (D, 1):
+            raise ValueError(f"{nm}: expected [num_slots, {Hkv}, {D}] with contiguous rows")
 
 
 def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -51,16 +75,13 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
     ks = _rows(k, Hkv, D, "k")
     vs = _rows(v, Hkv, D, "v")
     n = k.numel() // (Hkv * D)
-    for t, nm in ((k_cache, "k_cache"), (v_cache, "v_cache")):
-        if t.dim() != 3 or t.shape[1:] != (Hkv, D) or t.stride(2) != 1 or t.stride(1) != D:
-            raise ValueError(f"{nm}: expected [num_slots, {Hkv}, {D}] with contiguous rows")
+    _cache_rows(k_cache, v_cache, Hkv, D)
     if k_cache.stride(0) != v_cache.stride(0) or k_cache.shape[0] != v_cache.shape[0]:
         raise ValueError("k_cache and v_cache must have the same shape and slot stride")
-    sm = slot_mapping.reshape(-1)
+    sm = slot_mapping if slot_mapping.dim() == 1 else slot_mapping.reshape(-1)
     if sm.dtype != torch.int64 or sm.numel() != n or not sm.is_contiguous():
         raise ValueError("slot_mapping must be contiguous int64 with one entry per token")
-    cs = cos.reshape(-1, cos.shape[-1])
-    sn = sin.reshape(-1, sin.shape[-1])
+    cs, sn = _table(cos), _table(sin)
     if cs.stride(-1) != 1 or sn.stride(-1) != 1 or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin must have contiguous rows of equal stride")
     if cs.dtype != k.dtype or sn.dtype != k.dtype:
@@ -80,7 +101,7 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
         qos = _rows(q_out, Hq, D, "q_out")
     rr = None
     if rope_rows is not None:
-        rr = rope_rows.reshape(-1).to(torch.int64).contiguous()
+        rr = _index_rows(rope_rows)
     dev = k.device
     lib = _lib.load()
     _lib.check(lib.gllm_rope_kv_write(
@@ -133,18 +154,21 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     bf16 MFMA), always take the unfused path.
     """
     hidden = x.shape[-1]
-    xs = x.reshape(-1, hidden)
+    xs = x if x.dim() == 2 else x.reshape(-1, hidden)
     if xs.stride(-1) != 1:
         raise ValueError("x rows must be contiguous")
     n = xs.shape[0]
     for t, nm in ((k_cache, "k_cache"), (v_cache, "v_cache")):
-        if t.dim() != 3 or t.stride(2) != 1 or t.stride(1) != t.shape[2]:
+        if t.dim() != 3 or t.stride()[1:] != (t.shape[2], 1):
             raise ValueError(f"{nm}: expected [num_slots, Hkv, D] with contiguous rows")
     if k_cache.shape != v_cache.shape or k_cache.stride(0) != v_cache.stride(0):
         raise ValueError("k_cache and v_cache must have the same shape and slot stride")
-    Hkv, D = k_cache.shape[1], k_cache.shape[2]
-    for w, nm in ((w_k, "w_k"), (w_v, "w_v")) + (((w_q, "w_q"),) if w_q is not None else ()):
-        if w.dim() != 2 or w.shape[1] != hidden or w.stride(1) != 1 or w.dtype != x.dtype:
+    _, Hkv, D = k_cache.shape
+    for w, nm in ((w_k, "w_k"), (w_v, "w_v"), (w_q, "w_q")):
+        if w is None and nm == "w_q":
+            continue
+        shape = w.shape
+        if len(shape) != 2 or shape[1] != hidden or w.stride(1) != 1 or w.dtype != x.dtype:
             raise ValueError(f"{nm}: expected [heads * D, {hidden}] with contiguous rows in the model dtype")
     if w_k.shape[0] != Hkv * D or w_v.shape[0] != Hkv * D:
         raise ValueError("w_k / w_v must have num_kv_heads * head_dim rows")
@@ -155,13 +179,13 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
         Hq = w_q.shape[0] // D
         if q_out is None:
             q_out = torch.empty(n, Hq, D, dtype=x.dtype, device=x.device)
-        if q_out.reshape(-1, Hq * D).shape[0] != n or q_out.stride(-1) != 1:
+        if not (q_out.is_contiguous() and q_out.numel() == n * Hq * D) and (
+                q_out.reshape(-1, Hq * D).shape[0] != n or q_out.stride(-1) != 1):
             raise ValueError("q_out must hold one contiguous row of Hq * D per token")
-    sm = slot_mapping.reshape(-1)
+    sm = slot_mapping if slot_mapping.dim() == 1 else slot_mapping.reshape(-1)
     if sm.dtype != torch.int64 or sm.numel() != n or not sm.is_contiguous():
         raise ValueError("slot_mapping must be contiguous int64 with one entry per token")
-    cs = cos.reshape(-1, cos.shape[-1])
-    sn = sin.reshape(-1, sin.shape[-1])
+    cs, sn = _table(cos), _table(sin)
     if cs.stride(-1) != 1 or sn.stride(-1) != 1 or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin must have contiguous rows of equal stride")
     if cs.dtype != x.dtype or sn.dtype != x.dtype:
@@ -175,7 +199,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
         tps = n // ql.numel()
     rr = None
     if rope_rows is not None:
-        rr = rope_rows.reshape(-1).to(torch.int64).contiguous()
+        rr = _index_rows(rope_rows)
     if (unfused_from is not None and n >= unfused_from) or D not in (64, 128) or x.dtype != torch.bfloat16:
         k = F.linear(xs, w_k).view(n, Hkv, D)
         v = F.linear(xs, w_v).view(n, Hkv, D)
@@ -187,7 +211,9 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
             q_out.view(n, Hq, D).copy_(q)
         return q_out
     lib = _lib.load()
-    qrow = q_out.reshape(-1, Hq * D).stride(0) if q_out is not None else 0
+    qrow = 0
+    if q_out is not None:
+        qrow = Hq * D if q_out.is_contiguous() else q_out.reshape(-1, Hq * D).stride(0)
     wsb = lib.gllm_qkv_workspace_bytes(n, hidden, max(Hq, 1), Hkv, D, int(w_q is not None)) if split_k else 0
     # per call, from the caching allocator: calls on other streams have their own
     ws = torch.empty(wsb, dtype=torch.uint8, device=x.device) if wsb else None
@@ -208,8 +234,7 @@ def rope_rotate(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
     xs = _rows(x, H, D, "x")
     out = torch.empty_like(x, memory_format=torch.contiguous_format)
     n = x.numel() // (H * D)
-    cs = cos.reshape(-1, cos.shape[-1])
-    sn = sin.reshape(-1, sin.shape[-1])
+    cs, sn = _table(cos), _table(sin)
     rr = None if rope_rows is None else rope_rows.reshape(-1).to(torch.int64).contiguous()
     if cs.shape[-1] < D // 2 or (rr is None and cs.shape[0] < n) or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin need one row of at least D/2 entries per token")
@@ -305,6 +330,7 @@ class AttentionPlan:
         # facts every launch checks, computed once (a plan serves every layer of a step)
         self.rows = self._info["rows"]
         self.max_seq_len = max(sl, default=0)
+        self.max_query_len = max(ql, default=0)
         self.table_width = -(-self.max_seq_len // block_size)
 
     @property
@@ -326,14 +352,14 @@ def fused_kv_write_ok(plan: AttentionPlan, kv_dtype: torch.dtype) -> bool:
     """Whether :func:`paged_attention` can take ``kv_new`` for this plan and
     cache dtype: every sequence on the decode path of the kernel that runs
     (MFMA kernels: query_len x G <= 16; generic kernel: query_len <= 16)."""
-    if not plan.query_lens:
+    if not plan.max_query_len:             # no sequences
         return False
     mfma = (plan.dtype in (torch.bfloat16, torch.float16) and plan.head_dim in (64, 128)
             and kv_dtype in (plan.dtype, torch.float8_e4m3fn))
     G = plan.num_q_heads // plan.num_kv_heads
     if mfma:
-        return max(plan.query_lens) * G <= 16
-    return max(plan.query_lens) <= 16
+        return plan.max_query_len * G <= 16
+    return plan.max_query_len <= 16
 
 
 def paged_attention(plan: AttentionPlan, q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -356,20 +382,21 @@ def paged_attention(plan: AttentionPlan, q: torch.Tensor, k_cache: torch.Tensor,
     qs = _rows(q, Hq, D, "q")
     if out is None:
         out = torch.empty_like(q, memory_format=torch.contiguous_format)
-    os_ = _rows(out, Hq, D, "out")
+        os_ = Hq * D
+    else:
+        os_ = _rows(out, Hq, D, "out")
     if q.dtype != plan.dtype or out.dtype != plan.dtype:
         raise ValueError("q/out dtype differs from the plan's")
-    for t, nm in ((k_cache, "k_cache"), (v_cache, "v_cache")):
-        if t.dim() != 3 or t.shape[1:] != (Hkv, D) or t.stride(2) != 1 or t.stride(1) != D:
-            raise ValueError(f"{nm}: expected [num_slots, {Hkv}, {D}] with contiguous rows")
+    _cache_rows(k_cache, v_cache, Hkv, D)
     if k_cache.stride(0) != v_cache.stride(0):
         raise ValueError("k_cache and v_cache slot strides differ")
-    if block_table.dtype != torch.int32 or block_table.dim() != 2 or block_table.stride(1) != 1:
+    bt_shape = block_table.shape
+    if block_table.dtype != torch.int32 or len(bt_shape) != 2 or block_table.stride(1) != 1:
         raise ValueError("block_table must be int32 [B, W] with contiguous rows")
-    if block_table.shape[0] < len(plan.query_lens):
+    if bt_shape[0] < len(plan.query_lens):
         raise ValueError("block_table has fewer rows than the plan's sequences")
-    if block_table.shape[1] < plan.table_width:
-        raise ValueError(f"block_table width {block_table.shape[1]} < {plan.table_width} blocks the longest "
+    if bt_shape[1] < plan.table_width:
+        raise ValueError(f"block_table width {bt_shape[1]} < {plan.table_width} blocks the longest "
                          "sequence needs")
     rows = q.numel() // (Hq * D)
     if rows < plan.rows:
@@ -380,8 +407,7 @@ def paged_attention(plan: AttentionPlan, q: torch.Tensor, k_cache: torch.Tensor,
     if rope is not None:
         cos, sin, m = rope
         mode = {"position": _lib.ROPE_BY_POSITION, "row": _lib.ROPE_BY_ROW}[m]
-        cos = cos.reshape(-1, cos.shape[-1])
-        sin = sin.reshape(-1, sin.shape[-1])
+        cos, sin = _table(cos), _table(sin)
         if cos.stride(-1) != 1 or sin.stride(-1) != 1 or cos.stride(0) != sin.stride(0):
             raise ValueError("cos/sin must have contiguous rows of equal stride")
         if cos.dtype != q.dtype:
@@ -392,7 +418,7 @@ def paged_attention(plan: AttentionPlan, q: torch.Tensor, k_cache: torch.Tensor,
         cos_p, sin_p, rs = cos.data_ptr(), sin.data_ptr(), cos.stride(0)
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     num_blocks = k_cache.shape[0] // plan.block_size
-    lib = _lib.load()
+    lib = plan._lib
     if kv_new is not None:
         kn, vn = kv_new
         if kn.dtype != q.dtype or vn.dtype != q.dtype:

@@ -25,7 +25,7 @@ SOURCES = ["paged_attention.hip", "paged_attention_f16.hip", "api.hip", "rope_kv
 GENERIC = {"generic_attention.hip", "generic_attention_bf16.hip", "generic_attention_f16.hip"}
 NO_CONTRACT = {"rope_kv_write.hip", "qkv_proj.hip"} | GENERIC
 # MFMA accumulators stay in VGPRs (no per-tile AGPR<->VGPR copies)
-EXTRA = {f: ["-mllvm", "--amdgpu-mfma-vgpr-form"] for f in {"paged_attention.hip", "paged_attention_f16.hip"} | GENERIC}
+EXTRA = {f: ["-mllvm", "--amdgpu-mfma-vgpr-form"] for f in {"paged_attention.hip", "paged_attention_f16.hip", "qkv_proj.hip"} | GENERIC}
 COMMON = [
     f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC",
     # packed fp32 VALU ops are disabled on purpose for every HIP unit

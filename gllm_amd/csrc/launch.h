@@ -169,6 +169,8 @@ struct QKVArgs {
   int32_t cus;                   // compute units (planning)
   int32_t split_chunk, split_count;
   int32_t vec_stores;            // set by the launcher: rows aligned for 4-element stores
+  // large tiles: 256-token tiles and their workgroups, then 128-token tiles
+  int32_t full_tiles, full_wgs, half_tiles;
 };
 
 size_t qkv_workspace_bytes(int64_t num_tokens, int hidden, int heads, int head_dim, int cus);

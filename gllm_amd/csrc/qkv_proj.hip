@@ -26,6 +26,7 @@
 // take one launch with the whole hidden dimension per workgroup
 // (qkv_small_kernel).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "launch.h"
@@ -79,6 +80,137 @@ __device__ __forceinline__ void wait_stages(int after) {
       return;
     }
     wait_stages<IPS, M - 1>(after);
+  }
+}
+
+// Rounds, rotates and stores one wave's 32 tokens x one head of C: lane holds
+// C[token tbase + 8(j/4) + j%4][dim 32 b + lane % 32] in acc[b][j] (tbase
+// carries the lane's half).  Every per-token load (slot, cos/sin row, query
+// length) and every cos/sin value is issued before the first store (the stores
+// may alias them, so the compiler would otherwise serialise a round trip per
+// token).
+template <int D, bool KV8>
+__device__ __forceinline__ void qkv_store_rows(const QKVArgs& a, int kind, int h, int64_t tbase, int lane,
+                                               const f32x16* acc) {
+  constexpr int NB = D / 32, NH = NB / 2;
+  const int64_t N = a.num_tokens;
+  const int n = lane & 31;
+  const bool rope = kind == 1 || (kind == 0 && a.rotate_q);
+  int64_t dst[16];            // store offset per token (elements), -1: not written
+  uint32_t csn[16][NH];       // cos (low 16 bits) and sin (high) of the lane's rotation pairs
+  {
+    // loads first, each kind in its own loop (the conditions are uniform) and
+    // with the token index clamped into the batch, so they are in flight together
+    int64_t tc[16], crow[16], slot[16];
+    int32_t qlen[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      tc[j] = min(tbase + 8 * (j / 4) + (j % 4), N - 1);
+      crow[j] = tc[j];
+      slot[j] = 0;
+      qlen[j] = 0x7fffffff;
+    }
+    if (rope && a.rope_rows) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) crow[j] = a.rope_rows[tc[j]];
+    }
+    if (kind != 0) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) slot[j] = a.slot_mapping[tc[j]];
+    }
+    if (a.query_lens) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) qlen[j] = a.query_lens[tc[j] / a.tokens_per_seq];
+      // padded rows read cos/sin row 0 (their own position may lie past the
+      // table in mixed batches) and are not written below
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (tc[j] % a.tokens_per_seq >= qlen[j]) crow[j] = 0;
+    }
+    if (rope) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const uint16_t* cp = (const uint16_t*)a.cos + crow[j] * a.rope_row_stride + n;
+        const uint16_t* sp = (const uint16_t*)a.sin + crow[j] * a.rope_row_stride + n;
+#pragma unroll
+        for (int b = 0; b < NH; ++b) csn[j][b] = (uint32_t)cp[32 * b] | ((uint32_t)sp[32 * b] << 16);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int64_t tok = tbase + 8 * (j / 4) + (j % 4);
+      int64_t d = -1;
+      // padded rows of the reference's [B, T_q] layout are not written (q
+      // included); slots outside the pool are never addressed
+      const bool real = !a.query_lens || tok % a.tokens_per_seq < qlen[j];
+      if (tok < N && real) {
+        if (kind == 0) {
+          if (a.q_out) d = tok * a.q_out_row_stride + (int64_t)h * D;
+        } else {
+          if (slot[j] >= 0 && slot[j] < a.num_slots) d = slot[j] * a.cache_slot_stride + (int64_t)h * D;
+        }
+      }
+      dst[j] = d;
+    }
+  }
+  char* base = (char*)(kind == 0 ? a.q_out : (kind == 1 ? a.k_cache : a.v_cache));
+  const bool to_cache = kind != 0;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    float v[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b += 2) {                              // F.linear's bf16 output
+      v[b] = acc[b][j];
+      v[b + 1] = acc[b + 1][j];
+      round2_bf16(v[b], v[b + 1]);
+    }
+    if (rope) {
+#pragma unroll
+      for (int b = 0; b < NH; ++b)
+        rope_pair_bf16(v[b], v[b + NH], bf16_bits_to_f32(csn[j][b] & 0xffffu), bf16_bits_to_f32(csn[j][b] >> 16));
+    }
+    // Lanes n .. n + 3 hold head dims 32b + n .. + 3 of the same token: the
+    // quad gathers them (before the row test: every lane of a quad shares the
+    // token) and its first lane stores them with one 4-byte (fp8) or 8-byte
+    // (bf16) store.
+    uint32_t w[NB][2];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (KV8 && to_cache) {
+        const uint32_t x = pack_fp8x4(v[b], 0.f, 0.f, 0.f) & 0xffu;
+        const uint32_t y = x | (quad_xor1(x) << 8);
+        w[b][0] = y | (quad_xor2(y) << 16);
+        w[b][1] = 0u;
+      } else {
+        const uint32_t x = pack_bf16x2(v[b], 0.f) & 0xffffu;
+        const uint32_t y = x | (quad_xor1(x) << 16);
+        w[b][0] = y;
+        w[b][1] = quad_xor2(y);
+      }
+    }
+    if (dst[j] < 0) continue;
+    if (a.vec_stores) {                  // rows 4-element aligned (checked on the host)
+      if (n & 3) continue;
+      if (KV8 && to_cache) {
+        char* cp = base + dst[j];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) *reinterpret_cast<uint32_t*>(cp + 32 * b + n) = w[b][0];
+      } else {
+        char* cp = base + dst[j] * 2;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) st8(cp + (32 * b + n) * 2, u32x2{w[b][0], w[b][1]});
+      }
+    } else if (KV8 && to_cache) {
+      char* cp = base + dst[j];
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        *reinterpret_cast<uint8_t*>(cp + 32 * b + n) = (uint8_t)(pack_fp8x4(v[b], 0.f, 0.f, 0.f) & 0xffu);
+    } else {
+      char* cp = base + dst[j] * 2;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        *reinterpret_cast<uint16_t*>(cp + (32 * b + n) * 2) = (uint16_t)pack_bf16x2(v[b], 0.f);
+    }
   }
 }
 
@@ -207,133 +339,248 @@ qkv_rope_write_kernel(QKVArgs a) {
     }
   }
   if (!wact) return;
+#pragma unroll
+  for (int r = 0; r < RB; ++r)
+    qkv_store_rows<D, KV8>(a, kind, h, tok0 + tg * 32 * RB + 32 * r + 4 * hi, lane, acc[r]);
+}
 
-  // Epilogue: lane holds C[token 8(j/4) + 4 hi + j%4][dim 32 b + lane % 32].
-  // Every per-token load (slot, cos/sin row, query length) and every cos/sin
-  // value is issued before the first store (the stores may alias them, so
-  // the compiler would otherwise serialise a round trip per token).
-  const int n = lane & 31;
+// ------------------------------------------------------------------ large tiles
+// Prompt-sized batches: 256 tokens x 256 columns (256 / D consecutive heads of
+// one kind) per 8-wave workgroup, one per CU; each wave 64 tokens x 128 columns
+// as C^T blocks (W rows are the A operand, tokens the MFMA columns).  Bound: the
+// matrix cores, if LDS reads and copies stay off their path:
+//   * K slices of 64 (whole 128-byte lines per row) in a 2-stage ring, 128 KB;
+//   * a slice is four 16-wide steps; each step's six operand reads are placed
+//     between the eight MFMAs of the step before it, and the barrier that
+//     publishes the next slice stands before the last step's MFMAs, so its
+//     first reads and the next copies run under them;
+//   * the rounded C tile goes through the drained ring to the store pass, where
+//     a thread rotates and stores 8 + 8 dims of one (token, head) with 16-byte
+//     accesses.
+// Measured with the K / V write included (us; the 128- and 256-token kernel above
+// / three hipBLASLt GEMMs + the write kernel / this): 8B layer 2048 tokens 125 /
+// 126 / 97, 6000 324 / 278 / 271, 19,679 1200 / 946 / 834 (1188 TFLOP/s); 1B
+// layer 4096 tokens 84 / 79 / 56, 19,679 - / 283 / 231.  Four waves of 128 x 128
+// (fewer LDS reads per MFMA, one wave per SIMD) were 5-12% slower; spreading the
+// copies over two steps, wave priorities and a bare barrier are within 1%: at
+// ~110 us a round the card's clock under matrix load is what is left.
+constexpr int kTCols = 256;             // columns per workgroup
+// One tile: TM = 256 tokens, or 128 (the launch's last round, below): waves as
+// TM / 64 token groups x 512 / TM column groups.
+template <int D, bool KV8, int TM>
+__device__ __forceinline__ void qkv_tile_body(const QKVArgs& a, int64_t tok0, int head, char* lds) {
+  constexpr int HP = kTCols / D;          // heads per workgroup
+  constexpr int ROWB = 128;               // LDS bytes per X / W row of a slice
+  constexpr int XP = TM * ROWB;           // one X slice
+  constexpr int WP = kTCols * ROWB;       // one W slice
+  constexpr int WB = 2 * XP;              // LDS: X slices 0, 1, W slices 0, 1
+  constexpr int NT = 512;
+  constexpr int TG = TM / 64, CG = 8 / TG;               // wave grid
+  constexpr int NXB = TM / TG / 32;       // 32-token blocks per wave
+  constexpr int NWB = kTCols / CG / 32;   // 32-column blocks per wave
+  constexpr int RPC = NT / 8;             // rows per copy
+  constexpr int IX = TM / RPC, NI = IX + kTCols / RPC;   // copies per thread and slice: X, all
+  constexpr int NM = NXB * NWB, NR = NXB + NWB;          // MFMAs and operand reads of a 16-wide step
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t N = a.num_tokens;
+  const int kind = head < a.num_q_heads ? 0 : (head < a.num_q_heads + a.num_kv_heads ? 1 : 2);   // q, k, v
+  const int h0 = kind == 0 ? head : (kind == 1 ? head - a.num_q_heads : head - a.num_q_heads - a.num_kv_heads);
+  const char* w = (const char*)(kind == 0 ? a.w_q : (kind == 1 ? a.w_k : a.w_v));
+  const int64_t wstride = 2 * (kind == 0 ? a.w_q_row_stride : (kind == 1 ? a.w_k_row_stride : a.w_v_row_stride));
+  w += (int64_t)h0 * D * wstride;
+  const char* x = (const char*)a.x + tok0 * a.x_row_stride * 2;
+  const int nk = a.hidden / 64;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+
+  // copy i of a slice (X first, then W): rows 64 i + tid / 8, physical chunk
+  // tid % 8, which holds logical chunk (tid % 8) ^ (row & 7)
+  const int crow = tid >> 3, clc = (tid & 7) ^ (crow & 7);
+  uint32_t xoff[IX];
+#pragma unroll
+  for (int i = 0; i < IX; ++i)            // rows past the batch re-read the last token
+    xoff[i] = (uint32_t)(min((int64_t)(crow + RPC * i), N - 1 - tok0) * a.x_row_stride * 2) + clc * 16;
+  const uint32_t woff = (uint32_t)(crow * wstride) + clc * 16;
+  const int64_t wrpc = RPC * wstride;
+  auto copy = [&](int ks, int stage, int i) {
+    const bool isx = i < IX;
+    const char* base = (isx ? x : w + (i - IX) * wrpc) + (int64_t)ks * 128;
+    const uint32_t dst = lds0 + (isx ? stage * XP + i * NT * 16 : WB + stage * WP + (i - IX) * NT * 16) + wave * 1024;
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(isx ? xoff[isx ? i : 0] : woff), "s"(base),
+                 "s"(dst)
+                 : "memory", "m0");
+  };
+
+  const int tg = wave / CG, cg = wave % CG;       // token group (64), column group (256 / CG)
+  const int n = lane & 31, hi = lane >> 5;
+  int xk[4], wk[4];                               // operand chunk of 16-wide step kk
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    const int c = ((2 * kk + hi) ^ (n & 7)) << 4;
+    xk[kk] = (tg * 32 * NXB + n) * ROWB + c;
+    int v = WB + (cg * 32 * NWB + n) * ROWB + c;  // opaque: the W region's start cannot ride in the immediate
+    asm volatile("" : "+v"(v));
+    wk[kk] = v;
+  }
+  f32x16 acc[NWB][NXB];
+#pragma unroll
+  for (int b = 0; b < NWB; ++b)
+#pragma unroll
+    for (int r = 0; r < NXB; ++r) acc[b][r] = f32x16{};
+  u32x4 fw[2][NWB], fx[2][NXB];                     // operands of the current and the next step
+  // operand read q of step kk: the X blocks, then the W blocks
+  auto rd = [&](int stage, int kk, int p, int q) {
+    if (q < NXB) fx[p][q] = ld16(lds + stage * XP + 4096 * q + xk[kk]);
+    else fw[p][q - NXB] = ld16(lds + stage * WP + 4096 * (q - NXB) + wk[kk]);
+  };
+  auto mm = [&](int p, int i) {                   // MFMA i of a step
+    const int b = i / NXB, r = i % NXB;
+    acc[b][r] = mfma32(__builtin_bit_cast(bf16x8, fw[p][b]), __builtin_bit_cast(bf16x8, fx[p][r]), acc[b][r]);
+  };
+
+#pragma unroll
+  for (int i = 0; i < NI; ++i) copy(0, 0, i);
+  wait_vmcnt<0>();
+  __syncthreads();
+  if (nk > 1) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) copy(1, 1, i);
+  }
+#pragma unroll
+  for (int q = 0; q < NR; ++q) rd(0, 0, 0, q);
+  // slice ks in `stage`; more: there is a next slice to read, copies: one to copy
+  auto slice = [&](auto stage_, int ks, auto more, auto copies) {
+    constexpr int stage = decltype(stage_)::value;
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk) {
+#pragma unroll
+      for (int i = 0; i < NM; ++i) {
+        mm(kk & 1, i);
+#pragma unroll
+        for (int q = i * NR / NM; q < (i + 1) * NR / NM; ++q) rd(stage, kk + 1, (kk + 1) & 1, q);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    // every read of this slice is issued; the next slice's copies have landed
+    wait_vmcnt<0>();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NM; ++i) {
+      mm(1, i);
+#pragma unroll
+      for (int q = i * NR / NM; q < (i + 1) * NR / NM; ++q)
+        if (more) rd(stage ^ 1, 0, 0, q);
+#pragma unroll
+      for (int c = i * NI / NM; c < (i + 1) * NI / NM; ++c)
+        if (copies) copy(ks + 2, stage, c);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  const std::integral_constant<int, 0> s0;
+  const std::integral_constant<int, 1> s1;
+  int ks = 0;
+  for (; ks + 3 < nk; ks += 2) {                  // no branch between the MFMAs
+    slice(s0, ks, std::true_type(), std::true_type());
+    slice(s1, ks + 1, std::true_type(), std::true_type());
+  }
+  for (; ks < nk; ks += 2) {
+    slice(s0, ks, ks + 1 < nk, ks + 2 < nk);
+    if (ks + 1 < nk) slice(s1, ks + 1, ks + 2 < nk, ks + 3 < nk);
+  }
+  // C tile -> LDS, rounded to bf16 like F.linear's output: token rows of 512
+  // bytes, 16-byte chunk c of row t at c ^ (t & 31) (the lanes of a store hold
+  // 32 rows of one column)
+#pragma unroll
+  for (int b = 0; b < NWB; ++b)
+#pragma unroll
+    for (int r = 0; r < NXB; ++r) {
+      const int t = 32 * (tg * NXB + r) + n;
+#pragma unroll
+      for (int jq = 0; jq < 4; ++jq) {            // columns 32 (cg NWB + b) + 8 jq + 4 hi .. + 3
+        const int c = 4 * (cg * NWB + b) + jq;
+        st8(lds + t * 512 + ((c ^ (t & 31)) << 4) + 8 * hi,
+            u32x2{pack_bf16x2(acc[b][r][4 * jq], acc[b][r][4 * jq + 1]),
+                  pack_bf16x2(acc[b][r][4 * jq + 2], acc[b][r][4 * jq + 3])});
+      }
+    }
+  __syncthreads();
+  constexpr int PC = D / 16;                      // chunk pairs per head: dims 8p .. + 7 and D/2 + 8p ..
   const bool rope = kind == 1 || (kind == 0 && a.rotate_q);
-  constexpr int NH = NB / 2;
-#pragma unroll
-  for (int r = 0; r < RB; ++r) {
-  const int64_t tbase = tok0 + tg * 32 * RB + 32 * r + 4 * hi;
-  int64_t dst[16];            // store offset per token (elements), -1: not written
-  uint32_t csn[16][NH];       // cos (low 16 bits) and sin (high) of the lane's rotation pairs
-  {
-    // loads first, each kind in its own loop (the conditions are uniform) and
-    // with the token index clamped into the batch, so they are in flight together
-    int64_t tc[16], crow[16], slot[16];
-    int32_t qlen[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      tc[j] = min(tbase + 8 * (j / 4) + (j % 4), N - 1);
-      crow[j] = tc[j];
-      slot[j] = 0;
-      qlen[j] = 0x7fffffff;
-    }
-    if (rope && a.rope_rows) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) crow[j] = a.rope_rows[tc[j]];
-    }
-    if (kind != 0) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) slot[j] = a.slot_mapping[tc[j]];
-    }
-    if (a.query_lens) {
-#pragma unroll
-      for (int j = 0; j < 16; ++j) qlen[j] = a.query_lens[tc[j] / a.tokens_per_seq];
-      // padded rows read cos/sin row 0 (their own position may lie past the
-      // table in mixed batches) and are not written below
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        if (tc[j] % a.tokens_per_seq >= qlen[j]) crow[j] = 0;
-    }
+  for (int e = tid; e < TM * HP * PC; e += NT) {
+    const int t = e / (HP * PC), hp = (e / PC) % HP, pc = e % PC;
+    const int64_t tok = tok0 + t;
+    if (tok >= N) break;
+    if (a.query_lens && tok % a.tokens_per_seq >= a.query_lens[tok / a.tokens_per_seq]) continue;   // padded row
+    const int c = hp * (D / 8) + pc;
+    const char* row = lds + t * 512;
+    u32x4 lo = ld16(row + ((c ^ (t & 31)) << 4)), hc = ld16(row + (((c + PC) ^ (t & 31)) << 4));
     if (rope) {
+      const int64_t cr = a.rope_rows ? a.rope_rows[tok] : tok;
+      const u32x4 cw = ld16((const uint16_t*)a.cos + cr * a.rope_row_stride + 8 * pc);
+      const u32x4 sw = ld16((const uint16_t*)a.sin + cr * a.rope_row_stride + 8 * pc);
+      float x1[8], x2[8], cv[8], sv[8];
+      unpack_bf16x8(lo, x1);
+      unpack_bf16x8(hc, x2);
+      unpack_bf16x8(cw, cv);
+      unpack_bf16x8(sw, sv);
 #pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const uint16_t* cp = (const uint16_t*)a.cos + crow[j] * a.rope_row_stride + n;
-        const uint16_t* sp = (const uint16_t*)a.sin + crow[j] * a.rope_row_stride + n;
-#pragma unroll
-        for (int b = 0; b < NH; ++b) csn[j][b] = (uint32_t)cp[32 * b] | ((uint32_t)sp[32 * b] << 16);
-      }
+      for (int i = 0; i < 8; ++i) rope_pair_bf16(x1[i], x2[i], cv[i], sv[i]);
+      lo = pack8<__bf16>(x1);
+      hc = pack8<__bf16>(x2);
     }
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int64_t tok = tbase + 8 * (j / 4) + (j % 4);
-      int64_t d = -1;
-      // padded rows of the reference's [B, T_q] layout are not written (q
-      // included); slots outside the pool are never addressed
-      const bool real = !a.query_lens || tok % a.tokens_per_seq < qlen[j];
-      if (tok < N && real) {
-        if (kind == 0) {
-          if (a.q_out) d = tok * a.q_out_row_stride + (int64_t)h * D;
-        } else {
-          if (slot[j] >= 0 && slot[j] < a.num_slots) d = slot[j] * a.cache_slot_stride + (int64_t)h * D;
-        }
-      }
-      dst[j] = d;
+    const int d = 8 * pc;
+    if (kind == 0) {
+      uint16_t* op = (uint16_t*)a.q_out + tok * a.q_out_row_stride + (int64_t)(h0 + hp) * D + d;
+      st16(op, lo);
+      st16(op + D / 2, hc);
+      continue;
     }
-  }
-  char* base = (char*)(kind == 0 ? a.q_out : (kind == 1 ? a.k_cache : a.v_cache));
-  const bool to_cache = kind != 0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    float v[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b += 2) {                              // F.linear's bf16 output
-      v[b] = acc[r][b][j];
-      v[b + 1] = acc[r][b + 1][j];
-      round2_bf16(v[b], v[b + 1]);
-    }
-    if (rope) {
-#pragma unroll
-      for (int b = 0; b < NH; ++b)
-        rope_pair_bf16(v[b], v[b + NH], bf16_bits_to_f32(csn[j][b] & 0xffffu), bf16_bits_to_f32(csn[j][b] >> 16));
-    }
-    // Lanes n .. n + 3 hold head dims 32b + n .. + 3 of the same token: the
-    // quad gathers them (before the row test: every lane of a quad shares the
-    // token) and its first lane stores them with one 4-byte (fp8) or 8-byte
-    // (bf16) store.
-    uint32_t w[NB][2];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (KV8 && to_cache) {
-        const uint32_t x = pack_fp8x4(v[b], 0.f, 0.f, 0.f) & 0xffu;
-        const uint32_t y = x | (quad_xor1(x) << 8);
-        w[b][0] = y | (quad_xor2(y) << 16);
-        w[b][1] = 0u;
-      } else {
-        const uint32_t x = pack_bf16x2(v[b], 0.f) & 0xffffu;
-        const uint32_t y = x | (quad_xor1(x) << 16);
-        w[b][0] = y;
-        w[b][1] = quad_xor2(y);
-      }
-    }
-    if (dst[j] < 0) continue;
-    if (a.vec_stores) {                  // rows 4-element aligned (checked on the host)
-      if (n & 3) continue;
-      if (KV8 && to_cache) {
-        char* cp = base + dst[j];
-#pragma unroll
-        for (int b = 0; b < NB; ++b) *reinterpret_cast<uint32_t*>(cp + 32 * b + n) = w[b][0];
-      } else {
-        char* cp = base + dst[j] * 2;
-#pragma unroll
-        for (int b = 0; b < NB; ++b) st8(cp + (32 * b + n) * 2, u32x2{w[b][0], w[b][1]});
-      }
-    } else if (KV8 && to_cache) {
-      char* cp = base + dst[j];
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        *reinterpret_cast<uint8_t*>(cp + 32 * b + n) = (uint8_t)(pack_fp8x4(v[b], 0.f, 0.f, 0.f) & 0xffu);
+    const int64_t slot = a.slot_mapping[tok];
+    if (slot < 0 || slot >= a.num_slots) continue;
+    char* cp = (char*)(kind == 1 ? a.k_cache : a.v_cache);
+    const int64_t off = slot * a.cache_slot_stride + (int64_t)(h0 + hp) * D + d;
+    if constexpr (KV8) {
+      float v[8];
+      unpack_bf16x8(lo, v);
+      st8(cp + off, u32x2{pack_fp8x4(v[0], v[1], v[2], v[3]), pack_fp8x4(v[4], v[5], v[6], v[7])});
+      unpack_bf16x8(hc, v);
+      st8(cp + off + D / 2, u32x2{pack_fp8x4(v[0], v[1], v[2], v[3]), pack_fp8x4(v[4], v[5], v[6], v[7])});
     } else {
-      char* cp = base + dst[j] * 2;
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-        *reinterpret_cast<uint16_t*>(cp + (32 * b + n) * 2) = (uint16_t)pack_bf16x2(v[b], 0.f);
+      st16(cp + 2 * off, lo);
+      st16(cp + 2 * (off + D / 2), hc);
     }
   }
+}
+
+// The launch: token tiles of 256, then the last tokens in tiles of 128.  A round
+// is one workgroup per CU, so a last round that is nearly empty costs a whole
+// one; half tiles (0.55 of a round) fill it.  Workgroup b runs on XCD b % 8:
+// each XCD takes an equal share of the (tile, column group) pairs, neighbours in
+// blocks of gh groups x tiles, so the pairs it holds at once share their X and W
+// slices in its L2 and no XCD runs a round more than the others.
+struct QKVPair { int tile, group; };
+__device__ __forceinline__ bool qkv_pair(int b, int tiles, int ngroups, int gh, QKVPair& p) {
+  const int total = tiles * ngroups, xcd = b % kXcds, j = b / kXcds;
+  const int first = (int)((int64_t)total * xcd / kXcds), last = (int)((int64_t)total * (xcd + 1) / kXcds);
+  if (first + j >= last) return false;
+  const int per = tiles * gh, gb = (first + j) / per, rem = first + j - gb * per;
+  p.tile = rem / gh;
+  p.group = gb * gh + rem % gh;
+  return true;
+}
+
+template <int D, bool KV8>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) qkv_tile_kernel(QKVArgs a) {
+  __shared__ __attribute__((aligned(16))) char lds[2 * 2 * 256 * 128];
+  constexpr int HP = kTCols / D;
+  const int ngroups = (a.num_q_heads + 2 * a.num_kv_heads) / HP;
+  const int gh = ngroups % 8 == 0 ? 8 : (ngroups % 4 == 0 ? 4 : (ngroups % 2 == 0 ? 2 : 1));
+  QKVPair p;
+  if ((int)blockIdx.x < a.full_wgs) {
+    if (qkv_pair(blockIdx.x, a.full_tiles, ngroups, gh, p))
+      qkv_tile_body<D, KV8, 256>(a, (int64_t)p.tile * 256, p.group * HP, lds);
+  } else if (qkv_pair(blockIdx.x - a.full_wgs, a.half_tiles, ngroups, gh, p)) {
+    qkv_tile_body<D, KV8, 128>(a, (int64_t)a.full_tiles * 256 + (int64_t)p.tile * 128, p.group * HP, lds);
   }
 }
 
@@ -735,6 +982,26 @@ size_t qkv_workspace_bytes(int64_t n, int hidden, int heads, int head_dim, int c
 constexpr bool kTileBK64 = true, kTileBig64 = true;
 constexpr int kTileNS = 2;
 
+// Tiles of 256 and of 128 tokens for a batch, and how long they take in rounds
+// of full tiles (one workgroup per CU; a half tile takes kHalfRound of one).
+constexpr double kHalfRound = 0.55;
+struct QKVTiles { int64_t full, half; double rounds; };
+static QKVTiles qkv_tiles(int64_t n, int ngroups, int cus) {
+  const int64_t halves = (n + 127) / 128;
+  QKVTiles best{0, 0, 0.0};
+  // as many full tiles as whole rounds hold, one round fewer, or all of them
+  const int64_t per = std::max<int64_t>(1, cus / ngroups), all = (n + 255) / 256, fit = n / 256;
+  const int64_t r = std::min(fit * ngroups / cus, fit / per + 1);
+  for (int64_t c = 0; c < 3; ++c) {
+    const int64_t full = c == 2 ? all : std::max<int64_t>(0, std::min(fit, (r - c) * cus / ngroups));
+    const int64_t half = c == 2 ? 0 : halves - 2 * full;
+    const int64_t fw = full * ngroups, hw = half * ngroups;
+    const int64_t fr = (fw + cus - 1) / cus, spare = fr * cus - fw;   // half tiles start in the full ones' last round
+    const double t = (double)fr + kHalfRound * (double)((std::max<int64_t>(0, hw - spare) + cus - 1) / cus);
+    if (c == 0 || t < best.rounds) best = QKVTiles{full, half, t};
+  }
+  return best;
+}
 hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
   if (a.num_tokens == 0) return hipSuccess;
   const int64_t tiles = (a.num_tokens + 127) / 128;
@@ -788,6 +1055,38 @@ hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
       return hipErrorInvalidValue;
     }
     return hipGetLastError();
+  }
+  // Large batches: 256-column tiles (heads that pair within q and within k/v,
+  // whole 16-byte chunks everywhere)
+  const auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  const int hp = kTCols / a.head_dim;
+  if ((a.head_dim == 64 || a.head_dim == 128) && a.hidden % 64 == 0 && b.num_q_heads % hp == 0 &&
+      a.num_kv_heads % hp == 0 && a.num_tokens < (int64_t(1) << 30) && a.x_row_stride < (1 << 20) &&
+      std::max({a.w_q_row_stride, a.w_k_row_stride, a.w_v_row_stride}) < (1 << 20) && al16(a.k_cache) &&
+      al16(a.v_cache) && a.cache_slot_stride % 16 == 0 && al16(a.cos) && al16(a.sin) && a.rope_row_stride % 8 == 0 &&
+      (!a.q_out || (al16(a.q_out) && a.q_out_row_stride % 8 == 0))) {
+    const int ngroups = heads / hp;
+    const QKVTiles t = qkv_tiles(a.num_tokens, ngroups, a.cus);
+    // below 2 / 5 of the CUs the 128-token x one-head tiles spread the work wider
+    // (1B layer, us, these / those: 1024 tokens, 96 workgroups, 33.0 / 29.8; 1536,
+    // 144 workgroups, 33.8 / 51.2; 8B 700 tokens, 144 workgroups, 60.5 / 71.0)
+    if (5 * (t.full + t.half) * ngroups >= 2 * a.cus) {
+      const auto wgs_of = [&](int64_t tiles) { return (tiles * ngroups + kXcds - 1) / kXcds * kXcds; };
+      b.full_tiles = (int32_t)t.full;
+      b.half_tiles = (int32_t)t.half;
+      b.full_wgs = (int32_t)wgs_of(t.full);
+      const int64_t wgs = b.full_wgs + wgs_of(t.half);
+      if (wgs > 0x7fffffff) return hipErrorInvalidValue;
+      const dim3 grid((unsigned)wgs), block(512);
+      if (a.head_dim == 64) {
+        if (kv8) hipLaunchKernelGGL((qkv_tile_kernel<64, true>), grid, block, 0, st, b);
+        else hipLaunchKernelGGL((qkv_tile_kernel<64, false>), grid, block, 0, st, b);
+      } else {
+        if (kv8) hipLaunchKernelGGL((qkv_tile_kernel<128, true>), grid, block, 0, st, b);
+        else hipLaunchKernelGGL((qkv_tile_kernel<128, false>), grid, block, 0, st, b);
+      }
+      return hipGetLastError();
+    }
   }
   // 128-token tiles, one head each, in XCD-grouped order (a head's token
   // tiles share its W slice through one XCD's L2)

@@ -112,9 +112,10 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
 
 
 # Token count from which qkv_rope_kv_write projects with hipBLASLt (three
-# F.linear calls) and then runs the RoPE + KV write kernel: on MI355X the
-# fused kernel is ahead up to ~2k tokens (8B shapes: 4.3x at 64 tokens, 1.1x
-# at 2048) and behind from ~4k (0.90x at 4096, 0.82x at 19679 tokens).
+# F.linear calls) and then runs the RoPE + KV write kernel, where the 256-column
+# tiles do not take the batch (_tiles_ok): against the library those measure
+# 0.97-1.5x up to hidden 4096 (8B layer 19,679 tokens 834 us against 946) and
+# 0.86-1.14x at hidden 8192, whose wider GEMMs fill the GPU by themselves.
 QKV_UNFUSED_FROM = 3072
 
 
@@ -130,6 +131,17 @@ def qkv_fused_ok(x: torch.Tensor, w_q: torch.Tensor, w_k: torch.Tensor, w_v: tor
         return False
     return all(t.dtype == torch.bfloat16 and t.dim() == 2 and t.shape[1] == hidden and t.stride(1) == 1
                and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w_q, w_k, w_v))
+
+
+def _tiles_ok(hidden: int, Hq: int, Hkv: int, D: int, k_cache, v_cache, cos, sin, q_out) -> bool:
+    """Whether the projection's 256-column tiles take the call and are ahead of
+    the library at prompt sizes: heads that fill 256 columns within q and within
+    k / v, whole aligned 16-byte chunks, hidden up to 4096."""
+    if hidden % 64 or hidden > 4096 or D not in (64, 128) or (Hkv * D) % 256 or (Hq * D) % 256:
+        return False
+    if k_cache.stride(0) % 16 or cos.stride(0) % 8 or (q_out is not None and not q_out.is_contiguous()):
+        return False
+    return all(t is None or t.data_ptr() % 16 == 0 for t in (k_cache, v_cache, cos, sin, q_out))
 
 
 def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tensor, w_v: torch.Tensor,
@@ -148,8 +160,9 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     ``split_k``: let batches of few tokens split the hidden dimension over
     more workgroups (a device workspace); False forces the tile kernel.
     ``unfused_from``: from this many tokens the projections run as three
-    ``F.linear`` (hipBLASLt) followed by :func:`rope_kv_write`, which is faster
-    there; None runs the fused kernel at any size.  Head dims other than 64
+    ``F.linear`` (hipBLASLt) followed by :func:`rope_kv_write`, unless the fused
+    kernel's large tiles take the batch and are faster; None runs the fused
+    kernel at any size.  Head dims other than 64
     and 128, and models that are not bf16 (the fused kernel's projection is
     bf16 MFMA), always take the unfused path.
     """
@@ -200,7 +213,9 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     rr = None
     if rope_rows is not None:
         rr = _index_rows(rope_rows)
-    if (unfused_from is not None and n >= unfused_from) or D not in (64, 128) or x.dtype != torch.bfloat16:
+    if (D not in (64, 128) or x.dtype != torch.bfloat16 or unfused_from is not None and n >= unfused_from
+            and not (n >= QKV_UNFUSED_FROM and qkv_fused_ok(xs, w_k if w_q is None else w_q, w_k, w_v, k_cache, v_cache)
+                     and _tiles_ok(hidden, Hq, Hkv, D, k_cache, v_cache, cs, sn, q_out))):
         k = F.linear(xs, w_k).view(n, Hkv, D)
         v = F.linear(xs, w_v).view(n, Hkv, D)
         q = F.linear(xs, w_q).view(n, Hq, D) if w_q is not None else None

@@ -1256,9 +1256,11 @@ __global__ void __launch_bounds__(64 * kWaves) mixed_balanced_kernel(AttnArgs a)
 }
 
 // Prefill items only: kPrefillOnlyWaves-wave workgroups with a
-// kPrefillOnlyStages-stage ring.
+// kPrefillOnlyStages-stage ring.  D = 64: two workgroups per CU (128 registers,
+// 69 KB of LDS each), so one's start and barriers run under the other: 8
+// prompts of 512-4096 tokens, 32 / 8 heads, 328 -> 315 us.
 template <typename T, int D, bool KV8>
-__global__ void __launch_bounds__(64 * kPrefillOnlyWaves) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * kPrefillOnlyWaves) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
 prefill_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[PrefillCfg<D, kPrefillOnlyStages>::kLdsBytes];
   const WorkItem it = a.items[blockIdx.x];

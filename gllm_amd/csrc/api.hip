@@ -729,6 +729,23 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     if (!fills) best_hw = decode_heads_per_wg ? decode_heads_per_wg : 2;
     while (best_hw > 1 && best_hw / 2 >= num_kv_heads) best_hw /= 2;  // no idle head slots
     const int best_nw = 8;
+    const int64_t hg_n = (num_kv_heads + best_hw - 1) / best_hw;
+    // shortest split (a multiple of 32 keys, at least min_S) with at most n decode items
+    const auto shortest_split = [&](int64_t min_S, int64_t n) {
+      const auto items = [&](int64_t S) {
+        int64_t k = 0;
+        for (const SeqInfo& s : p->seqs)
+          if (s.q_len * G <= 16) k += (s.ctx_len + s.q_len + S - 1) / S * hg_n;
+        return k;
+      };
+      int64_t lo = min_S / 32, hi = cap / 32;     // items(S) falls as S grows
+      while (lo < hi) {
+        const int64_t mid = (lo + hi) / 2;
+        if (items(32 * mid) <= n) hi = mid;
+        else lo = mid + 1;
+      }
+      return 32 * lo;
+    };
     int64_t best_S = split_tokens < 0 ? 0 : split_tokens;
     if (best_S == 0) {
       if (fills) {
@@ -740,25 +757,14 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
         // keys, 8B heads: 208 items 21.4 us, 308 items 30.0, 132 items 25.7),
         // and shorter ones pay more start-up than they save.  In a mixed launch,
         // whose prefill items take CUs too, about half as many items as slots.
-        const int64_t hg = (num_kv_heads + best_hw - 1) / best_hw;
-        int64_t decode_tokens = 0;
-        for (const SeqInfo& s : p->seqs)
-          if (s.q_len * G <= 16) decode_tokens += s.ctx_len + s.q_len;
-        const auto items = [&](int64_t S) {
-          int64_t n = 0;
+        if (n_pf > 0) {
+          int64_t decode_tokens = 0;
           for (const SeqInfo& s : p->seqs)
-            if (s.q_len * G <= 16) n += ((s.ctx_len + s.q_len + S - 1) / S) * hg;
-          return n;
-        };
-        int64_t lo = 4, hi = cap / 32;     // in 32-key units; items(S) falls as S grows
-        while (lo < hi) {
-          const int64_t mid = (lo + hi) / 2;
-          if (items(32 * mid) <= cus) hi = mid;
-          else lo = mid + 1;
+            if (s.q_len * G <= 16) decode_tokens += s.ctx_len + s.q_len;
+          best_S = std::max<int64_t>(((2 * decode_tokens * hg_n + target - 1) / target + 31) / 32 * 32, 256);
+        } else {
+          best_S = shortest_split(128, cus);
         }
-        best_S = 32 * lo;
-        if (n_pf > 0)
-          best_S = std::max<int64_t>(((2 * decode_tokens * hg + target - 1) / target + 31) / 32 * 32, 256);
       }
     }
     best_S = std::min(best_S, cap);
@@ -770,16 +776,23 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     const int pw = ndec == 0 ? kPrefillOnlyWaves : 8;
     p->prefill_waves = pw;
     const int hgroups = (num_kv_heads + best_hw - 1) / best_hw;
-    const int64_t S = best_S;
-    p->split_len = (int32_t)S;
     p->head_groups = hgroups;
     p->merge.assign((size_t)num_seqs * hgroups, MergeInfo{0, 0});
     struct Keyed { int64_t work; WorkItem it; };
     std::vector<Keyed> pf, dc;
-    for (int i = 0; i < num_seqs; ++i) {
-      SeqInfo& s = p->seqs[i];
-      const int L = s.ctx_len + s.q_len;
-      if (s.q_len * G <= 16) {
+    // Longest work first so the tail is made of short items.
+    const auto longest_first = [](std::vector<Keyed>& v) {
+      std::stable_sort(v.begin(), v.end(), [](const Keyed& x, const Keyed& y) { return x.work > y.work; });
+    };
+    const auto decode_items = [&](int64_t S) {
+      p->split_len = (int32_t)S;
+      p->n_decode_seqs = 0;
+      p->n_partials = 0;
+      dc.clear();
+      for (int i = 0; i < num_seqs; ++i) {
+        SeqInfo& s = p->seqs[i];
+        const int L = s.ctx_len + s.q_len;
+        if (s.q_len * G > 16) continue;
         ++p->n_decode_seqs;
         // equal splits of 16-key multiples (a remainder split after full
         // S-key ones was the slowest item): len = ceil16(ceil(L / n)) for
@@ -798,24 +811,31 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
             dc.push_back({keys, WorkItem{kItemDecode | (hg << 8), i, sp, s.q_row_start, s.ctx_len, s.q_len,
                                          s.nsplits, s.partial_base}});
           }
-      } else {
-        ++p->n_prefill_seqs;
-        pcs.clear();
-        prefill_pieces(s, i, G, num_kv_heads, pcs, pw);
-        for (const PrefillPiece& pc : pcs) pf.push_back({pc.kend, pc.it});
       }
+      longest_first(dc);
+    };
+    decode_items(best_S);
+    for (int i = 0; i < num_seqs; ++i) {
+      if (p->seqs[i].q_len * G <= 16) continue;
+      ++p->n_prefill_seqs;
+      pcs.clear();
+      prefill_pieces(p->seqs[i], i, G, num_kv_heads, pcs, pw);
+      for (const PrefillPiece& pc : pcs) pf.push_back({pc.kend, pc.it});
     }
-    // Longest work first so the tail is made of short items.
-    std::stable_sort(pf.begin(), pf.end(), [](const Keyed& x, const Keyed& y) { return x.work > y.work; });
-    std::stable_sort(dc.begin(), dc.end(), [](const Keyed& x, const Keyed& y) { return x.work > y.work; });
+    longest_first(pf);
     // A decode-only batch of fewer than two items per CU whose items leave the
     // CUs unevenly loaded goes page-balanced: its partials and their merge cost
     // ~8 us, which a CU streams 256 KB in.  Measured (split / page-balanced us,
     // 8B heads; longest CU's excess over the mean): 48 sequences of 1100 keys
     // 57.4 / 50.3 (excess 275 KB), 32 of 500-3000 65.6 / 49.7 (660 KB), 40 of
     // 4000 161 / 121 (1.5 MB); 90 of 500-2000 92.3 / 94.5 (190 KB), 160 of
-    // 300-900 84.1 / 85.7 (210 KB).
-    if (pf.empty() && split_tokens == 0 && !decode_heads_per_wg && dc.size() < 2 * (size_t)cus) {
+    // 300-900 84.1 / 85.7 (210 KB).  In a mixed launch, where the prefill items
+    // fill most gaps, sequences are split at 1024 keys (three items per CU at
+    // most) instead, from an excess of 2 MB: 64 decodes of 512-4096 keys and two
+    // chunks 143 us unsplit, 113 so, 119 page-balanced (2.4 MB); 100 such decodes
+    // and four chunks 160 / 162 (1.5 MB), 100 of 200-1600 keys 59 / 69 (0.5 MB).
+    if (split_tokens == 0 && !decode_heads_per_wg && !dc.empty() && dc.size() < 2 * (size_t)cus &&
+        (pf.empty() || fills)) {
       std::vector<int64_t> load((size_t)cus, 0);   // min-heap of the CUs' keys, longest item first
       int64_t total = 0, longest = 0;
       for (const Keyed& k : dc) {
@@ -826,10 +846,14 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
         std::push_heap(load.begin(), load.end(), std::greater<int64_t>());
       }
       const int64_t key_bytes = (int64_t)best_hw * head_dim * 4;   // K and V, 16-bit
-      if ((longest - total / cus) * key_bytes > (int64_t(256) << 10)) {
-        p->n_partials = 0;
-        balanced = true;
-        plan_balanced_decode(p, cus, 0, 0);
+      if ((longest - total / cus) * key_bytes > (pf.empty() ? int64_t(256) << 10 : int64_t(2) << 20)) {
+        if (pf.empty()) {
+          p->n_partials = 0;
+          balanced = true;
+          plan_balanced_decode(p, cus, 0, 0);
+        } else {
+          decode_items(shortest_split(std::min<int64_t>(1024, cap), 3 * (int64_t)cus));
+        }
       }
     }
     if (!balanced) {

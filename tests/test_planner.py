@@ -46,5 +46,9 @@ def test_uneven_batches_go_page_balanced():
     assert _info([1] * 40, [4000] * 40)[0]["segs"] > 0           # 1.25 rounds of long items
     assert _info([1] * 32, uneven, split=1024)[0]["segs"] == 0   # a split length was asked for
     assert _info([1] * 31 + [64], uneven)[0]["segs"] == 0        # mixed batches only on request
+    # ... but a mixed batch whose decodes leave CUs far behind is split
+    skew = [r.randint(300, 600) for _ in range(56)] + [8000] * 8
+    assert _info([1] * 64 + [256], skew + [2000])[0]["split"] < 8000
+    assert _info([1] * 64 + [256], [600] * 64 + [2000])[0]["split"] > 600
     many = [r.randint(256, 4096) for _ in range(256)]
     assert _info([1] * 256, many)[0]["segs"] == 0                # four items per CU even out

@@ -764,6 +764,14 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
           best_S = std::max<int64_t>(((2 * decode_tokens * hg_n + target - 1) / target + 31) / 32 * 32, 256);
         } else {
           best_S = shortest_split(128, cus);
+          // The merge is a launch of its own: a split pays from 128 KB of K/V that
+          // the longest item sheds (unsplit / split us, 8 sequences of 224, 320,
+          // 448 keys: 1B heads 8.5 / 10.3, 9.6 / 10.3, 11.5 / 10.6; 8B heads 13.5 /
+          // 13.9, 15.8 / 13.8, 19.6 / 14.0).
+          int64_t longest = 0;
+          for (const SeqInfo& s : p->seqs) longest = std::max<int64_t>(longest, s.ctx_len + s.q_len);
+          const int64_t n = (longest + best_S - 1) / best_S;
+          if ((longest - (longest + n - 1) / n) * best_hw * head_dim * 4 < 128 << 10) best_S = cap;
         }
       }
     }

@@ -29,12 +29,22 @@ def test_small_batches_get_one_item_per_cu(L, D):
     i, nbytes = _info([1] * len(L), L, D=D)
     assert i["segs"] == 0 and i["dec"] == len(L)
     assert i["items"] <= CUS
+    if i["partials"] == 0:               # a split would shed less than 128 KB of K/V from the longest item
+        assert i["items"] == len(L) * -(-8 // i["hw"])
+        return
     # splits of at least 128 keys, and no coarser than the CUs ask for
     assert i["split"] >= 128
     if i["split"] > 128:
         finer = sum(-(-x // (i["split"] - 32)) for x in L) * -(-8 // i["hw"])
         assert finer > CUS
     assert nbytes >= i["partials"] * 16 * (D + 2) * 4
+
+
+@pytest.mark.parametrize("D,last_whole,first_split", [(64, 320, 448), (128, 192, 320)])
+@pytest.mark.parametrize("B", [1, 8, 16])
+def test_short_sequences_stay_whole(B, D, last_whole, first_split):
+    assert _info([1] * B, [last_whole] * B, D=D)[0]["partials"] == 0
+    assert _info([1] * B, [first_split] * B, D=D)[0]["partials"] > 0
 
 
 def test_uneven_batches_go_page_balanced():

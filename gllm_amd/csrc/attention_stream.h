@@ -3,7 +3,7 @@
 // models whose head dim the MFMA kernels do not take (not 64 or 128; up to
 // 256), and for a 16-bit model over a cache of another dtype (f32, or the
 // other 16-bit type).  Batches that fill the GPU with 128-column workgroups
-// run on attention_tile.hip.  fp32 arithmetic on v_mfma_f32_16x16x4_f32 with
+// run on attention_tile.h.  fp32 arithmetic on v_mfma_f32_16x16x4_f32 with
 // an exact online softmax (expf).  Compiled with -ffp-contract=off so the q
 // rotation rounds each op like the reference
 // (gllm/model/layers/attention.py:105-118): in fp32, or to the 16-bit model

@@ -544,7 +544,6 @@ int gllm_qkv_rope_kv_write(const void* x, int64_t x_row_stride, int64_t num_toke
 // kernel stores every element before the finish kernel sums them), so no
 // clearing is needed.
 namespace {
-constexpr size_t kQkvScratchBytes = size_t(24) << 20;
 constexpr int kMaxDevices = 64;
 __device__ __align__(256) char g_qkv_scratch[kQkvScratchBytes];
 void* g_qkv_scratch_ptr[kMaxDevices] = {};

@@ -7,6 +7,9 @@
 
 namespace gllm {
 
+// Scratch of the no-alloc QKV entry point (split-K partials)
+constexpr size_t kQkvScratchBytes = size_t(24) << 20;
+
 enum : int32_t { kF32 = 0, kBF16 = 1, kFP8 = 2, kF16 = 3 };   // kFP8: OCP e4m3fn (KV cache only)
 
 struct RopeKVWriteArgs {

@@ -951,25 +951,52 @@ constexpr int kQkvPartialBK = 64, kQkvPartialNS = 2;
 
 // Split-K plan for a batch: chunk length (multiple of 32, >= 256) and count,
 // or count 1 when the tile kernel already has enough workgroups.
-static void qkv_split_plan(int64_t n, int hidden, int heads, int cus, int* chunk, int* count) {
+static void qkv_split_plan(int64_t n, int hidden, int heads, int head_dim, int cus, int* chunk, int* count) {
   *chunk = hidden;
   *count = 1;
   const int64_t tiles = (n + 127) / 128;
   if (n == 0 || tiles * heads >= cus || hidden < 512) return;
-  const int64_t wgs64 = ((n + 63) / 64) * heads;
-  int64_t want = (2 * (int64_t)cus + wgs64 - 1) / wgs64;           // about two workgroups per CU
-  want = std::min<int64_t>(std::min<int64_t>(want, hidden / 256), 16);   // the finish kernel sums <= 16 chunks
-  if (want <= 1) return;
+  const int64_t tiles64 = (n + 63) / 64, wgs64 = tiles64 * heads;
   const int g = hidden % kQkvPartialBK == 0 ? kQkvPartialBK : 32;   // chunks in whole k-steps of the partial kernel
-  const int c = (int)(((hidden + want - 1) / want + g - 1) / g * g);
-  *chunk = c;
-  *count = (hidden + c - 1) / c;
+  const int most = std::min(hidden / 256, 16);                      // the finish kernel sums <= 16 chunks
+  const auto chunk_of = [&](int c) { return ((hidden + c - 1) / c + g - 1) / g * g; };
+  int want = (int)std::min<int64_t>((2 * (int64_t)cus + wgs64 - 1) / wgs64, most);   // about two workgroups per CU
+  if (head_dim == 128 && want > 1) {
+    // The partial kernel is bound by the L2s its workgroups share: the time goes
+    // with the workgroups per CU of the fullest XCD (super-groups are dealt out
+    // whole; fewer than two per CU wait on their loads), times a chunk and a
+    // start of ~200 k; a chunk's partials cost n x heads x D / 5000 of the same
+    // unit (~9 ns).  Another count is taken where that is 5% shorter and its
+    // partials fit the no-alloc entry point's scratch.  Measured (us, about two
+    // workgroups per CU -> so): hidden 4096, 48 heads, 96 / 128 / 256 / 320 tokens
+    // 24.9 / 27.5 / 39.7 / 51.5 -> 22.4 / 24.6 / 36.1 / 44.7; hidden 3072, 40
+    // heads, 96 / 192 / 256 tokens 21.2 / 25.9 / 30.2 -> 18.4 / 23.7 / 26.4; at
+    // head dim 64 the counts around two per CU are within 2%.
+    const auto cost = [&](int c) {
+      const int len = chunk_of(c), cc = (hidden + len - 1) / len;
+      const double per_cu = (double)(wgs64 * cc) / cus;
+      const int64_t nsg = n <= 64 ? kXcds : qkv_groups(tiles64, heads * cc, cus).nsg;
+      const double fullest = per_cu * (double)((nsg + kXcds - 1) / kXcds * kXcds) / (double)nsg;
+      return std::max(fullest, 4.0 - per_cu) * (len + 200) + cc * (double)(n * heads * head_dim) / 5000.0;
+    };
+    double best = 0.95 * cost(want);
+    for (int c = 2; c <= most; ++c) {
+      if (c > want && (size_t)c * n * heads * head_dim * sizeof(float) > kQkvScratchBytes) break;
+      if (const double t = cost(c); t < best) {
+        best = t;
+        want = c;
+      }
+    }
+  }
+  if (want <= 1) return;
+  *chunk = chunk_of(want);
+  *count = (hidden + *chunk - 1) / *chunk;
 }
 
 size_t qkv_workspace_bytes(int64_t n, int hidden, int heads, int head_dim, int cus) {
   if (qkv_small_cb(n, hidden, heads, head_dim, cus)) return 0;
   int chunk, count;
-  qkv_split_plan(n, hidden, heads, cus, &chunk, &count);
+  qkv_split_plan(n, hidden, heads, head_dim, cus, &chunk, &count);
   return count > 1 ? (size_t)count * n * heads * head_dim * sizeof(float) : 0;
 }
 
@@ -1028,7 +1055,7 @@ hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
     return hipGetLastError();
   }
   int chunk, count;
-  qkv_split_plan(a.num_tokens, a.hidden, heads, a.cus, &chunk, &count);
+  qkv_split_plan(a.num_tokens, a.hidden, heads, a.head_dim, a.cus, &chunk, &count);
   if (count > 1 && a.workspace &&
       a.workspace_bytes >= (size_t)count * a.num_tokens * heads * a.head_dim * sizeof(float)) {
     b.split_chunk = chunk;

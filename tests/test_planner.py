@@ -62,3 +62,18 @@ def test_uneven_batches_go_page_balanced():
     assert _info([1] * 64 + [256], [600] * 64 + [2000])[0]["split"] > 600
     many = [r.randint(256, 4096) for _ in range(256)]
     assert _info([1] * 256, many)[0]["segs"] == 0                # four items per CU even out
+
+
+@pytest.mark.parametrize("hidden,heads", [(4096, 32), (3072, 24), (5120, 40), (8192, 64), (2048, 16), (1024, 8)])
+def test_qkv_split_fits_the_noalloc_scratch(hidden, heads):
+    """A batch whose partials fit 24 MiB at about two workgroups per CU fits
+    them at the count that is chosen."""
+    lib = _lib.load()
+    for n in list(range(33, 700, 7)) + [256, 320, 512]:
+        F = (heads + 16) * 128
+        wgs = -(-n // 64) * (heads + 16)
+        want = min(-(-2 * CUS // wgs), hidden // 256, 16)
+        got = lib.gllm_qkv_workspace_bytes(n, hidden, heads, 8, 128, 1)
+        assert got % (n * F * 4) == 0 and got // (n * F * 4) <= 16
+        if want * n * F * 4 <= 24 << 20:
+            assert got <= 24 << 20, (n, got)

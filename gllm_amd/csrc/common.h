@@ -255,9 +255,18 @@ __device__ __forceinline__ u32x4 fp8x8_to(uint32_t w0, uint32_t w1) {
 // the kernel waits for its own copies with wait_vmcnt before the barrier that
 // publishes a stage.  M0 is set inside the asm and listed as clobbered (the
 // compiler warns that it reserves M0; in these kernels every M0 write in the
-// generated code is this asm's own, checked in the assembly).
+// generated code is this asm's own, checked in the assembly).  A copy may not
+// follow the scalar write of its M0 directly (one wait state, which the
+// hardware does not insert and the compiler does not add inside an asm): with
+// the old M0 it would land at the previous copy's place.
 __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds_base) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base)
+               : "memory", "m0");
+}
+// The same from a wave-uniform base and a 32-bit byte offset per lane.
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_base)
+               : "memory", "m0");
 }
 // s_waitcnt vmcnt(N) leaving the other counters alone (gfx9 encoding).
 template <int N>

@@ -406,9 +406,7 @@ __device__ __forceinline__ void qkv_tile_body(const QKVArgs& a, int64_t tok0, in
     const bool isx = i < IX;
     const char* base = (isx ? x : w + (i - IX) * wrpc) + (int64_t)ks * 128;
     const uint32_t dst = lds0 + (isx ? stage * XP + i * NT * 16 : WB + stage * WP + (i - IX) * NT * 16) + wave * 1024;
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(isx ? xoff[isx ? i : 0] : woff), "s"(base),
-                 "s"(dst)
-                 : "memory", "m0");
+    lds_dma16(base, isx ? xoff[isx ? i : 0] : woff, dst);
   };
 
   const int tg = wave / CG, cg = wave % CG;       // token group (64), column group (256 / CG)

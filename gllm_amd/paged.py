@@ -36,9 +36,10 @@ def _rows(t: torch.Tensor, heads: int, head_dim: int, name: str) -> int:
     return stride
 
 
-def _table(t: torch.Tensor) -> torch.Tensor:
-    """cos / sin as rows."""
-    return t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
+def _flat(t: torch.Tensor) -> torch.Tensor:
+    """The last dim as rows.  A single row goes through reshape too, which
+    replaces the stride it has from a wider tensor."""
+    return t if t.dim() == 2 and t.shape[0] != 1 else t.reshape(-1, t.shape[-1])
 
 
 def _index_rows(t: torch.Tensor) -> torch.Tensor:
@@ -81,7 +82,7 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
     sm = slot_mapping if slot_mapping.dim() == 1 else slot_mapping.reshape(-1)
     if sm.dtype != torch.int64 or sm.numel() != n or not sm.is_contiguous():
         raise ValueError("slot_mapping must be contiguous int64 with one entry per token")
-    cs, sn = _table(cos), _table(sin)
+    cs, sn = _flat(cos), _flat(sin)
     if cs.stride(-1) != 1 or sn.stride(-1) != 1 or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin must have contiguous rows of equal stride")
     if cs.dtype != k.dtype or sn.dtype != k.dtype:
@@ -167,7 +168,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     bf16 MFMA), always take the unfused path.
     """
     hidden = x.shape[-1]
-    xs = x if x.dim() == 2 else x.reshape(-1, hidden)
+    xs = _flat(x)
     if xs.stride(-1) != 1:
         raise ValueError("x rows must be contiguous")
     n = xs.shape[0]
@@ -198,7 +199,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     sm = slot_mapping if slot_mapping.dim() == 1 else slot_mapping.reshape(-1)
     if sm.dtype != torch.int64 or sm.numel() != n or not sm.is_contiguous():
         raise ValueError("slot_mapping must be contiguous int64 with one entry per token")
-    cs, sn = _table(cos), _table(sin)
+    cs, sn = _flat(cos), _flat(sin)
     if cs.stride(-1) != 1 or sn.stride(-1) != 1 or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin must have contiguous rows of equal stride")
     if cs.dtype != x.dtype or sn.dtype != x.dtype:
@@ -249,7 +250,7 @@ def rope_rotate(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
     xs = _rows(x, H, D, "x")
     out = torch.empty_like(x, memory_format=torch.contiguous_format)
     n = x.numel() // (H * D)
-    cs, sn = _table(cos), _table(sin)
+    cs, sn = _flat(cos), _flat(sin)
     rr = None if rope_rows is None else rope_rows.reshape(-1).to(torch.int64).contiguous()
     if cs.shape[-1] < D // 2 or (rr is None and cs.shape[0] < n) or cs.stride(0) != sn.stride(0):
         raise ValueError("cos/sin need one row of at least D/2 entries per token")
@@ -422,7 +423,7 @@ def paged_attention(plan: AttentionPlan, q: torch.Tensor, k_cache: torch.Tensor,
     if rope is not None:
         cos, sin, m = rope
         mode = {"position": _lib.ROPE_BY_POSITION, "row": _lib.ROPE_BY_ROW}[m]
-        cos, sin = _table(cos), _table(sin)
+        cos, sin = _flat(cos), _flat(sin)
         if cos.stride(-1) != 1 or sin.stride(-1) != 1 or cos.stride(0) != sin.stride(0):
             raise ValueError("cos/sin must have contiguous rows of equal stride")
         if cos.dtype != q.dtype:

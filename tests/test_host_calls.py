@@ -1,0 +1,53 @@
+"""Which kernel a Python call reaches and with what strides (no GPU: a recorder
+stands in for the library)."""
+import pytest
+import torch
+
+from gllm_amd import _lib, paged
+
+BF = torch.bfloat16
+
+
+class Recorder:
+    """Every entry point succeeds and is noted with its arguments."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append((name, args))
+            return 0
+        return call
+
+    def names(self):
+        return [n for n, _ in self.calls if n != "gllm_qkv_workspace_bytes"]
+
+
+@pytest.fixture
+def lib(monkeypatch):
+    rec = Recorder()
+    monkeypatch.setattr(_lib, "load", lambda: rec)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda dev: 0)
+    return rec
+
+
+def _caches(slots, Hkv, D, dtype=BF):
+    return torch.zeros(slots, Hkv, D, dtype=dtype), torch.zeros(slots, Hkv, D, dtype=dtype)
+
+
+def test_one_row_of_a_wider_table(lib):
+    """One cos / sin row, or one token row, cut out of wider rows is a whole row:
+    its stride means nothing."""
+    kc, vc = _caches(32, 4, 64)
+    wide, own = torch.zeros(9, 64, dtype=BF), torch.zeros(1, 32, dtype=BF)
+    cos, slots = wide[5:6, :32], torch.zeros(1, dtype=torch.int64)
+    assert cos.stride(0) != own.stride(0)
+    k = torch.zeros(1, 4, 64, dtype=BF)
+    paged.rope_kv_write(k, k, cos, own, kc, vc, slots)
+    paged.rope_rotate(k, cos, own)
+    x = torch.zeros(3, 260, dtype=BF)[:1, :256]          # rows 260 elements apart: no multiple of 8
+    w = torch.zeros(256, 256, dtype=BF)
+    paged.qkv_rope_kv_write(x, w, w, w, cos, own, kc, vc, slots)
+    name, args = lib.calls[-1]
+    assert name == "gllm_qkv_rope_kv_write" and args[1] == 256

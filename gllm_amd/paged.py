@@ -124,14 +124,14 @@ def qkv_fused_ok(x: torch.Tensor, w_q: torch.Tensor, w_k: torch.Tensor, w_v: tor
                  k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
     """Whether the fused kernels of :func:`qkv_rope_kv_write` take these rows,
     weights and caches: bf16 rows of a hidden size that is a multiple of 32, 16-byte
-    aligned, a bf16 or fp8 cache, head dim 64 or 128."""
+    aligned and not overlapping, a bf16 or fp8 cache, head dim 64 or 128."""
     hidden = x.shape[-1]
     if x.dim() != 2 or hidden % 32 or k_cache.shape[2] not in (64, 128):
         return False
     if k_cache.dtype not in (torch.bfloat16, torch.float8_e4m3fn) or v_cache.dtype != k_cache.dtype:
         return False
     return all(t.dtype == torch.bfloat16 and t.dim() == 2 and t.shape[1] == hidden and t.stride(1) == 1
-               and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w_q, w_k, w_v))
+               and t.stride(0) >= hidden and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w_q, w_k, w_v))
 
 
 def _tiles_ok(hidden: int, Hq: int, Hkv: int, D: int, k_cache, v_cache, cos, sin, q_out) -> bool:

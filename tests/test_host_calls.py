@@ -51,3 +51,24 @@ def test_one_row_of_a_wider_table(lib):
     paged.qkv_rope_kv_write(x, w, w, w, cos, own, kc, vc, slots)
     name, args = lib.calls[-1]
     assert name == "gllm_qkv_rope_kv_write" and args[1] == 256
+
+
+def _qkv(lib, n=paged.QKV_UNFUSED_FROM, x=None, **kw):
+    """A projection call that the large tiles take; the entry points it reached."""
+    hidden, H, D = 64, 4, 64
+    x = torch.zeros(n, hidden, dtype=BF) if x is None else x
+    w = torch.zeros(H * D, hidden, dtype=BF)
+    kc, vc = _caches(16, H, D)
+    tab, slots = torch.zeros(n, D // 2, dtype=BF), torch.zeros(n, dtype=torch.int64)
+    paged.qkv_rope_kv_write(x, w, w, w, tab, tab, kc, vc, slots, **kw)
+    return lib.names()
+
+
+def test_projection_of_expanded_rows(lib):
+    """Token rows that overlap (a row expanded) are the library's at prompt sizes:
+    the kernels refuse row strides below the hidden size."""
+    row = torch.zeros(1, 64, dtype=BF)
+    n = paged.QKV_UNFUSED_FROM
+    assert _qkv(lib) == ["gllm_qkv_rope_kv_write"]
+    lib.calls.clear()
+    assert _qkv(lib, x=row.expand(n, 64)) == ["gllm_rope_kv_write"]

@@ -120,6 +120,10 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
 QKV_UNFUSED_FROM = 3072
 
 
+class _Default(int):
+    """A threshold nobody asked for: the routing may set it aside."""
+
+
 def qkv_fused_ok(x: torch.Tensor, w_q: torch.Tensor, w_k: torch.Tensor, w_v: torch.Tensor,
                  k_cache: torch.Tensor, v_cache: torch.Tensor) -> bool:
     """Whether the fused kernels of :func:`qkv_rope_kv_write` take these rows,
@@ -149,7 +153,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
                       cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                       slot_mapping: torch.Tensor, *, rotate_q: bool = True, q_out: torch.Tensor | None = None,
                       query_lens: torch.Tensor | None = None, rope_rows: torch.Tensor | None = None,
-                      split_k: bool = True, unfused_from: int | None = QKV_UNFUSED_FROM):
+                      split_k: bool = True, unfused_from: int | None = _Default(QKV_UNFUSED_FROM)):
     """Fused ``linear_q/k/v`` + RoPE + KV-cache write of
     ``gllm/model/layers/attention.py:139-161`` (bf16 model).
 
@@ -161,9 +165,9 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     ``split_k``: let batches of few tokens split the hidden dimension over
     more workgroups (a device workspace); False forces the tile kernel.
     ``unfused_from``: from this many tokens the projections run as three
-    ``F.linear`` (hipBLASLt) followed by :func:`rope_kv_write`, unless the fused
-    kernel's large tiles take the batch and are faster; None runs the fused
-    kernel at any size.  Head dims other than 64
+    ``F.linear`` (hipBLASLt) followed by :func:`rope_kv_write`; by default from
+    QKV_UNFUSED_FROM where the fused kernel's large tiles do not take the batch;
+    None runs the fused kernel at any size.  Head dims other than 64
     and 128, and models that are not bf16 (the fused kernel's projection is
     bf16 MFMA), always take the unfused path.
     """
@@ -215,7 +219,8 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     if rope_rows is not None:
         rr = _index_rows(rope_rows)
     if (D not in (64, 128) or x.dtype != torch.bfloat16 or unfused_from is not None and n >= unfused_from
-            and not (n >= QKV_UNFUSED_FROM and qkv_fused_ok(xs, w_k if w_q is None else w_q, w_k, w_v, k_cache, v_cache)
+            and not (isinstance(unfused_from, _Default)
+                     and qkv_fused_ok(xs, w_k if w_q is None else w_q, w_k, w_v, k_cache, v_cache)
                      and _tiles_ok(hidden, Hq, Hkv, D, k_cache, v_cache, cs, sn, q_out))):
         k = F.linear(xs, w_k).view(n, Hkv, D)
         v = F.linear(xs, w_v).view(n, Hkv, D)

@@ -72,3 +72,15 @@ def test_projection_of_expanded_rows(lib):
     assert _qkv(lib) == ["gllm_qkv_rope_kv_write"]
     lib.calls.clear()
     assert _qkv(lib, x=row.expand(n, 64)) == ["gllm_rope_kv_write"]
+
+
+def test_explicit_threshold_forces_the_library(lib):
+    """A threshold the caller gives holds as it stands; only the default lets the
+    large tiles take prompts beyond it."""
+    n = paged.QKV_UNFUSED_FROM
+    for given in (n, int("3072"), 100, 1):
+        lib.calls.clear()
+        assert _qkv(lib, unfused_from=given) == ["gllm_rope_kv_write"], given
+    for kw in ({}, {"unfused_from": None}, {"unfused_from": n + 1}):
+        lib.calls.clear()
+        assert _qkv(lib, **kw) == ["gllm_qkv_rope_kv_write"], kw

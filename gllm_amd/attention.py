@@ -161,7 +161,7 @@ class Attention:
         if (x.dtype != torch.bfloat16 or n >= paged.QKV_UNFUSED_FROM
                 or not paged.qkv_fused_ok(x.view(n, -1) if x.is_contiguous() else x, wq, wk, wv, k_cache, v_cache)
                 or cos_pos.dtype != x.dtype or slots.dtype != torch.int64 or not slots.is_contiguous()
-                or slots.numel() != n):
+                or slots.numel() != n or slots.device != x.device or meta.query_lens.device != x.device):
             return None
         plan = self._plan(meta, x.dtype, x.device)
         if not paged.fused_kv_write_ok(plan, k_cache.dtype):

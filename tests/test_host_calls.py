@@ -3,6 +3,7 @@ stands in for the library)."""
 import pytest
 import torch
 
+import gllm_amd
 from gllm_amd import _lib, paged
 
 BF = torch.bfloat16
@@ -84,3 +85,53 @@ def test_explicit_threshold_forces_the_library(lib):
     for kw in ({}, {"unfused_from": None}, {"unfused_from": n + 1}):
         lib.calls.clear()
         assert _qkv(lib, **kw) == ["gllm_qkv_rope_kv_write"], kw
+
+
+class _Plan:
+    """What a layer asks of the step's plan (kept on the metadata)."""
+    block_size, dtype, max_query_len = 16, BF, 1
+
+    def __init__(self, Hq, Hkv, D):
+        self.num_q_heads, self.num_kv_heads, self.head_dim = Hq, Hkv, D
+
+
+def _forward(monkeypatch, cls=gllm_amd.Attention, rows=2, Hq=4, Hkv=2, D=64, dev="meta", slots_dev="meta", ql_dev="meta",
+             patch=None):
+    """The calls one decode step of a layer makes, tensors without storage."""
+    calls = []
+
+    def note(name, out):
+        def call(*args, **kw):
+            calls.append(name + ("+kv" if kw.get("kv_new") is not None else ""))
+            return out
+        return call
+
+    class Cfg:
+        num_attn_heads, num_kv_heads, head_dim, hidden_size, dtype = Hq, Hkv, D, Hq * D, BF
+
+    hid = Hq * D
+    w = {f"model.layers.0.self_attn.{n}_proj.weight": torch.zeros(h * D, hid, dtype=BF, device=dev)
+         for n, h in (("q", Hq), ("k", Hkv), ("v", Hkv), ("o", Hq))}
+    att = cls(0, Cfg, w)
+    out = torch.zeros(rows, 1, Hq, D, dtype=BF, device=dev)
+    monkeypatch.setattr(paged, "qkv_rope_kv_write", note("fused projection", out))
+    monkeypatch.setattr(paged, "paged_attention", note("attention", out))
+    if patch:
+        patch(att, note("override", out))
+    meta = gllm_amd.AttentionMetadata(
+        query_lens=torch.ones(rows, dtype=torch.int32, device=ql_dev), seq_lens=torch.ones(rows, dtype=torch.int32),
+        max_seq_len=1, block_table=torch.zeros(rows, 1, dtype=torch.int32, device=dev), slot_mapping=None,
+        query_slot_mapping=torch.zeros(rows, 1, dtype=torch.int64, device=slots_dev), bias=None, block_size=16)
+    meta._gllm_plan = _Plan(Hq, Hkv, D)
+    tab = torch.zeros(rows, 1, D // 2, dtype=BF, device=dev)
+    att.forward(torch.zeros(rows, 1, hid, dtype=BF, device=dev), tab, tab,
+                torch.zeros(2, 32, Hkv, D, dtype=BF, device=dev), meta)
+    return calls
+
+
+def test_forward_reads_no_host_metadata(monkeypatch):
+    """Slots and query lengths on the host stay with the route that takes the
+    slots from the block table: the fused projection reads both on the GPU."""
+    assert _forward(monkeypatch) == ["fused projection", "attention"]
+    assert _forward(monkeypatch, slots_dev="cpu") == ["attention+kv"]
+    assert _forward(monkeypatch, ql_dev="cpu") == ["attention+kv"]

@@ -135,3 +135,16 @@ def test_forward_reads_no_host_metadata(monkeypatch):
     assert _forward(monkeypatch) == ["fused projection", "attention"]
     assert _forward(monkeypatch, slots_dev="cpu") == ["attention+kv"]
     assert _forward(monkeypatch, ql_dev="cpu") == ["attention+kv"]
+
+
+def test_forward_reaches_an_overridden_attention(monkeypatch):
+    """A subclass's, or one object's, own ``attention`` is called on every step."""
+    class Own(gllm_amd.Attention):
+        def attention(self, *args):
+            self.seen = True
+            return super().attention(*args)
+
+    seen = []
+    assert _forward(monkeypatch, cls=Own, patch=lambda att, call: seen.append(att)) == ["attention+kv"]
+    assert seen[0].seen
+    assert _forward(monkeypatch, patch=lambda att, call: setattr(att, "attention", call)) == ["override"]

@@ -161,7 +161,7 @@ class Attention:
         k_cache, v_cache = kv_cache[0], kv_cache[1]
         slots = meta.query_slot_mapping
         n = x.shape[0] * x.shape[1]
-        if (x.dtype != torch.bfloat16 or n >= paged.QKV_UNFUSED_FROM
+        if (x.dtype != torch.bfloat16 or n >= paged.QKV_UNFUSED_FROM or k_cache.shape != v_cache.shape
                 or not paged.qkv_fused_ok(x.view(n, -1) if x.is_contiguous() else x, wq, wk, wv, k_cache, v_cache)
                 or cos_pos.dtype != x.dtype or slots.dtype != torch.int64 or not slots.is_contiguous()
                 or slots.numel() != n or slots.device != x.device or meta.query_lens.device != x.device):

@@ -96,7 +96,7 @@ class _Plan:
 
 
 def _forward(monkeypatch, cls=gllm_amd.Attention, rows=2, Hq=4, Hkv=2, D=64, dev="meta", slots_dev="meta", ql_dev="meta",
-             patch=None):
+             patch=None, pool=None):
     """The calls one decode step of a layer makes, tensors without storage."""
     calls = []
 
@@ -125,7 +125,7 @@ def _forward(monkeypatch, cls=gllm_amd.Attention, rows=2, Hq=4, Hkv=2, D=64, dev
     meta._gllm_plan = _Plan(Hq, Hkv, D)
     tab = torch.zeros(rows, 1, D // 2, dtype=BF, device=dev)
     att.forward(torch.zeros(rows, 1, hid, dtype=BF, device=dev), tab, tab,
-                torch.zeros(2, 32, Hkv, D, dtype=BF, device=dev), meta)
+                torch.zeros(2, 32, Hkv, D, dtype=BF, device=dev) if pool is None else pool, meta)
     return calls
 
 
@@ -148,3 +148,9 @@ def test_forward_reaches_an_overridden_attention(monkeypatch):
     assert _forward(monkeypatch, cls=Own, patch=lambda att, call: seen.append(att)) == ["attention+kv"]
     assert seen[0].seen
     assert _forward(monkeypatch, patch=lambda att, call: setattr(att, "attention", call)) == ["override"]
+
+
+def test_forward_takes_caches_of_unlike_length(monkeypatch):
+    """K and V pools given as a pair may differ in their number of slots."""
+    pool = tuple(torch.zeros(n, 2, 64, dtype=BF, device="meta") for n in (32, 48))
+    assert _forward(monkeypatch, pool=pool) == ["attention+kv"]

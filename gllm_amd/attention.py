@@ -97,6 +97,21 @@ def plan_for(meta, *, num_q_heads: int, num_kv_heads: int, head_dim: int,
     return plan
 
 
+def _fused_ahead(rows: int, hidden: int, cols: int) -> bool:
+    """Whether a decode step's fused projections (``cols`` output columns) beat
+    three ``F.linear``.  One layer's step from a graph, weights out of cache, 64
+    keys per sequence, linear / fused us (1, 64, 256, 512, 1024, 3000 rows): hidden
+    4096, 32 / 8 heads 55 / 25, 56 / 32, 86 / 72, 133 / 121, 233 / 222, 586 / 586;
+    hidden 2048, 32 / 8 heads of 64 31 / 13, 34 / 21, 44 / 32, 59 / 49, 97 / 89, 232 /
+    223.  Wider layers' own GEMMs fill the GPU sooner: hidden 8192, 64 / 8 heads
+    67 / 54, 75 / 64, 156 / 133, 207 / 231, 337 / 346, 851 / 836; hidden 6144 at 512
+    rows 172 / 193, hidden 5120 at 576 176 / 182; and with 24,576 columns (64 / 64
+    heads) no step is ahead (1 row 105 / 109, 33 rows 147 / 151)."""
+    if hidden <= 4096:
+        return rows < paged.QKV_UNFUSED_FROM
+    return rows <= 256 and cols <= 16384
+
+
 class Attention:
     """``attention.py:30-182``.  ``weights`` maps the reference's safetensors
     names (``model.layers.{i}.self_attn.{q,k,v,o}_proj.weight``) to tensors;
@@ -155,13 +170,14 @@ class Attention:
     def _fused_decode(self, x, wq, wk, wv, cos_pos, sin_pos, kv_cache, meta):
         """A bf16 decode step with the three projections, the RoPE and the KV
         write in the fused kernels (``attention.py:139-161``), then the
-        attention; None where they do not take the call.  The projections of a
-        decode batch are three launches of few workgroups otherwise (48 tokens
-        of an 8B layer: 42 us as three ``F.linear``, 21 fused)."""
+        attention; None where they do not take the call or are behind.  The
+        projections of a decode batch are three launches of few workgroups
+        otherwise (48 tokens of an 8B layer: 42 us as three ``F.linear``, 21 fused)."""
         k_cache, v_cache = kv_cache[0], kv_cache[1]
         slots = meta.query_slot_mapping
         n = x.shape[0] * x.shape[1]
-        if (x.dtype != torch.bfloat16 or n >= paged.QKV_UNFUSED_FROM or k_cache.shape != v_cache.shape
+        if (x.dtype != torch.bfloat16 or not _fused_ahead(n, self.hidden_size, wq.shape[0] + 2 * wk.shape[0])
+                or k_cache.shape != v_cache.shape
                 or not paged.qkv_fused_ok(x.view(n, -1) if x.is_contiguous() else x, wq, wk, wv, k_cache, v_cache)
                 or cos_pos.dtype != x.dtype or slots.dtype != torch.int64 or not slots.is_contiguous()
                 or slots.numel() != n or slots.device != x.device or meta.query_lens.device != x.device):

@@ -154,3 +154,16 @@ def test_forward_takes_caches_of_unlike_length(monkeypatch):
     """K and V pools given as a pair may differ in their number of slots."""
     pool = tuple(torch.zeros(n, 2, 64, dtype=BF, device="meta") for n in (32, 48))
     assert _forward(monkeypatch, pool=pool) == ["attention+kv"]
+
+
+def test_forward_projects_with_the_library_where_it_is_ahead(monkeypatch):
+    """Wide layers: the fused kernels for up to 256 rows, F.linear beyond."""
+    fused, linear = ["fused projection", "attention"], ["attention+kv"]
+    wide, wider = dict(Hq=64, Hkv=8, D=128), dict(Hq=64, Hkv=64, D=128)
+    assert _forward(monkeypatch, rows=256, **wide) == fused
+    for rows in (257, 512, 3000):
+        assert _forward(monkeypatch, rows=rows, **wide) == linear
+    assert _forward(monkeypatch, rows=1, **wider) == linear
+    for Hq in (16, 32):
+        assert _forward(monkeypatch, rows=3000, Hq=Hq, Hkv=8, D=128) == fused
+    assert _forward(monkeypatch, rows=paged.QKV_UNFUSED_FROM) == linear

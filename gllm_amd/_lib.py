@@ -48,6 +48,7 @@ SIGNATURES = {
                                                       _i32, _p, _p, _i64, _i64, _p, _p, _i64, _p, _p, _p, _i64, _i32,
                                                       _i32, _i32, _i32, _i32, _p]),
     "gllm_qkv_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32, _i32]),
+    "gllm_qkv_tiles_ahead": (ctypes.c_int, [_i64, _i32, _i32, _i32]),
     "gllm_attention_dense": (ctypes.c_int, [_p, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _p,
                                             _i64, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _p]),
 }

@@ -606,6 +606,13 @@ size_t gllm_qkv_workspace_bytes(int64_t num_tokens, int32_t hidden, int32_t num_
                              device_cus());
 }
 
+int gllm_qkv_tiles_ahead(int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim) {
+  if (num_tokens <= 0 || num_tokens >= (int64_t(1) << 30) || num_q_heads < 0 || num_q_heads > 65535 ||
+      num_kv_heads <= 0 || num_kv_heads > 65535 || (head_dim != 64 && head_dim != 128))
+    return 0;
+  return qkv_tiles_ahead(num_tokens, num_q_heads * head_dim, num_kv_heads * head_dim, device_cus()) ? 1 : 0;
+}
+
 int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const int32_t* seq_lens,
                           int32_t num_seqs, int64_t q_seq_stride, int32_t num_q_heads,
                           int32_t num_kv_heads, int32_t head_dim, int32_t block_size, int32_t dtype,

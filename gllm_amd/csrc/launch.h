@@ -177,6 +177,7 @@ struct QKVArgs {
 };
 
 size_t qkv_workspace_bytes(int64_t num_tokens, int hidden, int heads, int head_dim, int cus);
+bool qkv_tiles_ahead(int64_t num_tokens, int q_cols, int kv_cols, int cus);
 
 hipError_t launch_rope_kv_write(const RopeKVWriteArgs& a, hipStream_t stream);
 hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t stream);

@@ -26,6 +26,7 @@
 // take one launch with the whole hidden dimension per workgroup
 // (qkv_small_kernel).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -1027,6 +1028,37 @@ static QKVTiles qkv_tiles(int64_t n, int ngroups, int cus) {
   }
   return best;
 }
+
+// Whether a prompt batch's tiles are ahead of three library GEMMs and the RoPE +
+// KV write kernel.  Both run 256 x 256 tiles in rounds of one per CU, so each
+// side's time goes with its rounds: the tiles' over all columns together, the
+// library's over q, k and v by themselves, a GEMM of less than half (a quarter)
+// of a round taking 0.8 (0.4) of one in smaller tiles.  The library's rounds are
+// shorter by an eighth (hidden 4096: 93-105 us against 104-117), and a round of
+// the tiles' half tiles measures 0.62 here, so the tiles go first from 1.12 of
+// their rounds on.  Measured over 52 sizes of 3,072-19,700 tokens, us, library /
+// tiles (library rounds / tiles'): 32 / 8 heads of 128, hidden 4096: 4,100 tokens
+// 252 / 209 (1.40), 12,000 662 / 504 (1.08), 12,288 492 / 540 (1.03), 13,677 566 / 627
+// (1.02), 16,384 628 / 694 (1.00), 16,390 960 / 721 (1.38), 19,679 950 / 847 (1.19);
+// hidden 3072, 24 / 8 heads: 3,244 125 / 146 (0.97), 9,768 295 / 328 (1.04); 32 / 8
+// heads of 64, hidden 2048: 4,096 78 / 59 (1.81), 5,377 98 / 103 (0.97).  Of 292
+// points the rule gives 224 to the tiles, 223 of them no slower than 1% (17,906
+// tokens 763 / 793), and most of the others within 10% of a draw.
+constexpr double kLibraryRound = 1.12, kHalfRoundAhead = 0.62;
+bool qkv_tiles_ahead(int64_t n, int q_cols, int kv_cols, int cus) {
+  const int64_t tiles = (n + 255) / 256;
+  const auto gemm = [&](int cols) {
+    const double r = (double)(tiles * cols) / 256 / cus;
+    return cols == 0 ? 0.0 : r <= 0.25 ? 0.4 : r <= 0.5 ? 0.8 : std::ceil(r);
+  };
+  const int ngroups = (q_cols + 2 * kv_cols) / kTCols;
+  if (ngroups <= 0) return false;
+  const QKVTiles t = qkv_tiles(n, ngroups, cus);
+  const int64_t full = (t.full * ngroups + cus - 1) / cus, spare = full * cus - t.full * ngroups;
+  const int64_t half = (std::max<int64_t>(0, t.half * ngroups - spare) + cus - 1) / cus;
+  return gemm(q_cols) + 2 * gemm(kv_cols) >= kLibraryRound * ((double)full + kHalfRoundAhead * (double)half);
+}
+
 hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
   if (a.num_tokens == 0) return hipSuccess;
   const int64_t tiles = (a.num_tokens + 127) / 128;

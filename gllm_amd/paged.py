@@ -114,9 +114,7 @@ def rope_kv_write(k: torch.Tensor, v: torch.Tensor, cos: torch.Tensor, sin: torc
 
 # Token count from which qkv_rope_kv_write projects with hipBLASLt (three
 # F.linear calls) and then runs the RoPE + KV write kernel, where the 256-column
-# tiles do not take the batch (_tiles_ok): against the library those measure
-# 0.97-1.5x up to hidden 4096 (8B layer 19,679 tokens 834 us against 946) and
-# 0.86-1.14x at hidden 8192, whose wider GEMMs fill the GPU by themselves.
+# tiles do not take the batch or are behind (_tiles_ok).
 QKV_UNFUSED_FROM = 3072
 
 
@@ -138,15 +136,22 @@ def qkv_fused_ok(x: torch.Tensor, w_q: torch.Tensor, w_k: torch.Tensor, w_v: tor
                and t.stride(0) >= hidden and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (x, w_q, w_k, w_v))
 
 
-def _tiles_ok(hidden: int, Hq: int, Hkv: int, D: int, k_cache, v_cache, cos, sin, q_out) -> bool:
+def _tiles_ok(n: int, hidden: int, Hq: int, Hkv: int, D: int, k_cache, v_cache, cos, sin, q_out) -> bool:
     """Whether the projection's 256-column tiles take the call and are ahead of
     the library at prompt sizes: heads that fill 256 columns within q and within
-    k / v, whole aligned 16-byte chunks, hidden up to 4096."""
+    k / v, whole aligned 16-byte chunks, a token count whose tiles fill their
+    rounds (``gllm_qkv_tiles_ahead``, with the measurements), and hidden up to
+    4096: above it the two are level or alternate with the token count (3,072-19,679
+    tokens, library / fused time: hidden 4608 0.93-1.24, 5120 1.00-1.30, 6144
+    0.98-1.18, 7168 0.94-1.18, 8192 0.88-1.07).  Layers of few heads, which the
+    launcher gives to smaller tiles or the split, are ahead too (768 columns 1.3-2.3,
+    1,024 1.2-1.8)."""
     if hidden % 64 or hidden > 4096 or D not in (64, 128) or (Hkv * D) % 256 or (Hq * D) % 256:
         return False
     if k_cache.stride(0) % 16 or cos.stride(0) % 8 or (q_out is not None and not q_out.is_contiguous()):
         return False
-    return all(t is None or t.data_ptr() % 16 == 0 for t in (k_cache, v_cache, cos, sin, q_out))
+    return all(t is None or t.data_ptr() % 16 == 0 for t in (k_cache, v_cache, cos, sin, q_out)) \
+        and bool(_lib.load().gllm_qkv_tiles_ahead(n, Hq, Hkv, D))
 
 
 def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tensor, w_v: torch.Tensor,
@@ -221,7 +226,7 @@ def qkv_rope_kv_write(x: torch.Tensor, w_q: torch.Tensor | None, w_k: torch.Tens
     if (D not in (64, 128) or x.dtype != torch.bfloat16 or unfused_from is not None and n >= unfused_from
             and not (isinstance(unfused_from, _Default)
                      and qkv_fused_ok(xs, w_k if w_q is None else w_q, w_k, w_v, k_cache, v_cache)
-                     and _tiles_ok(hidden, Hq, Hkv, D, k_cache, v_cache, cs, sn, q_out))):
+                     and _tiles_ok(n, hidden, Hq, Hkv, D, k_cache, v_cache, cs, sn, q_out))):
         k = F.linear(xs, w_k).view(n, Hkv, D)
         v = F.linear(xs, w_v).view(n, Hkv, D)
         q = F.linear(xs, w_q).view(n, Hq, D) if w_q is not None else None

@@ -135,6 +135,12 @@ int gllm_qkv_rope_kv_write(const void* x, int64_t x_row_stride, int64_t num_toke
 size_t gllm_qkv_workspace_bytes(int64_t num_tokens, int32_t hidden, int32_t num_q_heads, int32_t num_kv_heads,
                                 int32_t head_dim, int32_t with_q);
 
+/* 1 where gllm_qkv_rope_kv_write is expected to finish a prompt batch (from
+ * about 3,072 tokens, hidden up to 4096) before three library GEMMs and
+ * gllm_rope_kv_write would, else 0: for callers that have both.  num_q_heads 0:
+ * K and V only.  Host arithmetic on the sizes; no counterpart in the reference. */
+int gllm_qkv_tiles_ahead(int64_t num_tokens, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim);
+
 /*
  * gllm_qkv_rope_kv_write without a workspace argument and without any
  * allocation (no hipMalloc/hipFree, no allocating library call).  No

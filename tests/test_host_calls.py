@@ -18,11 +18,11 @@ class Recorder:
     def __getattr__(self, name):
         def call(*args):
             self.calls.append((name, args))
-            return 0
+            return int(name == "gllm_qkv_tiles_ahead")
         return call
 
     def names(self):
-        return [n for n, _ in self.calls if n != "gllm_qkv_workspace_bytes"]
+        return [n for n, _ in self.calls if n not in ("gllm_qkv_workspace_bytes", "gllm_qkv_tiles_ahead")]
 
 
 @pytest.fixture

@@ -108,9 +108,12 @@ __device__ __forceinline__ u32x2 pack4(const Raw4<KV>& r) {
 //     already the B operand of step j; A is V[key 4grp + j][64u + 4n + e], so
 //     one 4-element load per (j, u) feeds the four output blocks e.
 // A 16-bit model's K, V and q are 16-bit values, so its S runs on the 16x16x32
-// instruction (products exact, fp32 sums) and P V on 16x16x16 with the fp32 p
-// split into two 16-bit parts (p = hi + lo to 2^-17 in bf16, 2^-22 in fp16):
-// head dim 256, one sequence of 2048 keys: 125 us with fp32 MFMA, 76 so.
+// instruction (products exact, fp32 sums).  P stays an fp32 value: in bf16, whose
+// exponents are fp32's, as the sum of three parts (24 bits) on 16x16x16; fp16
+// parts of a small p would be subnormal, so an fp16 model's P V runs on the fp32
+// instruction like an fp32 model's.  32 / 8 heads, us with P V in fp32 / three
+// parts (bf16): 1 x 2048 keys 48 / 43 at D = 96, 84 / 77 at 256; 64 x 2000 keys
+// 123 / 116 and 214 / 202; 2 x 300 rows 55 / 48 and 83 / 78.
 // The waves' (max, sum, acc) merge through LDS at the end.  Latency-bound at
 // short contexts (one round trip per PF sub-tiles), HBM-bound beyond.  Against
 // one workgroup per (query head, query row) with VALU dot products, which read
@@ -134,8 +137,9 @@ struct StreamCfg {
   template <bool FUSED> static constexpr int stage() { return (16 + (FUSED ? 32 : 0)) * kQS; }
   template <bool FUSED> static constexpr int lds() { return kMerge > stage<FUSED>() ? kMerge : stage<FUSED>(); }
   // sub-tiles in flight beside the current one (registers; at DP 256 the eight
-  // waves overlap each other's loads instead)
-  static constexpr int kPF = DP == 256 && kNW == 8 ? 0 : (VEC && kBytes <= 256 ? 2 : 1);
+  // waves overlap each other's loads instead; a 16-bit model's element loads
+  // leave no room for another one)
+  static constexpr int kPF = (DP == 256 && kNW == 8) || (!VEC && sizeof(QT) == 2) ? 0 : (VEC && kBytes <= 256 ? 2 : 1);
 };
 template <bool DENSE, typename KV, typename QT, int DP, bool FUSED, bool VEC>
 __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_stream_kernel(AttnArgs a) {
@@ -145,6 +149,7 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
   constexpr int NU = DP / 64;             // V column groups of 64 dims
   constexpr int QS = Cfg::kQS;
   constexpr bool k16 = sizeof(QT) == 2;   // 16-bit MFMA (above)
+  constexpr bool kSplitP = std::is_same<QT, __bf16>::value;   // p in three parts (above)
   // q of the columns, the new keys' K and V (FUSED); the merge reuses the area
   __shared__ __attribute__((aligned(16))) float lds[Cfg::template lds<FUSED>()];
   __shared__ float mml[NW][16][2];
@@ -370,10 +375,23 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
     l = l * alpha + ((s[0] + s[1]) + (s[2] + s[3]));
     m = mn;
     // the sub-tile's P V from zero, then one FMA per output with the rescale
-    if constexpr (k16) {
-      const u32x2 ph = {E16<QT>::pack2(s[0], s[1]), E16<QT>::pack2(s[2], s[3])};
-      const u32x2 pl = {E16<QT>::pack2(s[0] - E16<QT>::lo(ph[0]), s[1] - E16<QT>::hi(ph[0])),
-                        E16<QT>::pack2(s[2] - E16<QT>::lo(ph[1]), s[3] - E16<QT>::hi(ph[1]))};
+    auto rescale = [&](int u, int e, const f32x4& w) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[u][e][i] = __builtin_fmaf(o[u][e][i], alpha, w[i]);
+    };
+    if constexpr (kSplitP) {
+      // p = p0 + p1 + p2 in bf16: 24 bits, the low parts added first
+      u32x2 pp[3];
+      f32x4 r = s;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        pp[c] = u32x2{E16<QT>::pack2(r[0], r[1]), E16<QT>::pack2(r[2], r[3])};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          r[2 * i] -= E16<QT>::lo(pp[c][i]);
+          r[2 * i + 1] -= E16<QT>::hi(pp[c][i]);
+        }
+      }
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         u32x2 vv[4];
@@ -385,10 +403,9 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
           const u32x2 av = {__builtin_amdgcn_perm(vv[1][e / 2], vv[0][e / 2], sel),
                             __builtin_amdgcn_perm(vv[3][e / 2], vv[2][e / 2], sel)};
           f32x4 w = {0.f, 0.f, 0.f, 0.f};
-          w = E16<QT>::mfma16k16(av, pl, w);
-          w = E16<QT>::mfma16k16(av, ph, w);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[u][e][i] = __builtin_fmaf(o[u][e][i], alpha, w[i]);
+          for (int c = 2; c >= 0; --c) w = E16<QT>::mfma16k16(av, pp[c], w);
+          rescale(u, e, w);
         }
       }
     } else {
@@ -399,14 +416,18 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
         for (int e = 0; e < 4; ++e) w[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const f32x4 vv = vf(j, u);
+          f32x4 vv;
+          if constexpr (k16) {
+            const u32x2 x = vf(j, u);
+            vv = f32x4{E16<QT>::lo(x[0]), E16<QT>::hi(x[0]), E16<QT>::lo(x[1]), E16<QT>::hi(x[1])};
+          } else {
+            vv = vf(j, u);
+          }
 #pragma unroll
           for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[j], w[e], 0, 0, 0);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[u][e][i] = __builtin_fmaf(o[u][e][i], alpha, w[e][i]);
+        for (int e = 0; e < 4; ++e) rescale(u, e, w[e]);
       }
     }
   };

@@ -1,0 +1,75 @@
+"""Generic attention of 16-bit models where the last bits of the probabilities
+decide the result."""
+import math
+
+import pytest
+import torch
+
+from gllm_amd import paged
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+F32, BF, F16 = torch.float32, torch.bfloat16, torch.float16
+BS = 16
+
+
+def run(q, k, v, dtype, kv=None, kv_new=None):
+    """Every row of q [rows, Hq, D] over the keys k / v [n, Hkv, D] (the rows are
+    the last ones), in scattered blocks."""
+    n, Hkv, D = k.shape
+    rows, Hq = q.shape[:2]
+    nb = -(-n // BS)
+    table = torch.randperm(nb, generator=torch.Generator().manual_seed(n)).int() + 1
+    slot = table.long()[torch.arange(n) // BS] * BS + torch.arange(n) % BS
+    caches = []
+    for t in (k, v):
+        c = torch.zeros((nb + 1) * BS, Hkv, D, dtype=kv or dtype)
+        c[slot] = t.to(kv or dtype)
+        caches.append(c.to(DEV))
+    plan = paged.AttentionPlan([rows], [n], num_q_heads=Hq, num_kv_heads=Hkv, head_dim=D, block_size=BS, dtype=dtype,
+                               device=DEV)
+    new = None if kv_new is None else tuple(t.to(dtype).to(DEV) for t in kv_new)
+    return paged.paged_attention(plan, q.to(dtype).to(DEV), *caches, table.view(1, -1).to(DEV), kv_new=new).cpu()
+
+
+@pytest.mark.parametrize("D", [96, 256])
+@pytest.mark.parametrize("shift", [10, 17, 21, 23])
+def test_f16_small_weights(shift, D):
+    """One key takes almost all of the weight and has V = 0: the result is the
+    sum of 1,500 equal weights just above 2^-shift, an fp16 subnormal from shift
+    15 on.  fp32 weights: only the output's rounding is left."""
+    n, Hq = 1501, 4
+    g = torch.Generator().manual_seed(shift)
+    k = torch.zeros(n, 1, D)
+    q = torch.zeros(1, Hq, D)
+    q[..., 0] = torch.tensor([(shift - h / 5) * math.log(2) for h in range(Hq)]).half().float()
+    k[700, 0, 0] = math.sqrt(D)                      # score q[0] there, 0 elsewhere
+    k = k.half().float()
+    v = 1.0 + torch.rand(n, 1, D, generator=g).half().float()
+    v[700] = 0.0
+    out = run(q, k, v, F16).double()
+    s = (q[0].double() @ k[:, 0].double().t()) / math.sqrt(D)
+    ref = torch.softmax(s, -1) @ v[:, 0].half().double()
+    # one fp16 rounding, 2^-11 of the value (or half a subnormal step), and a few fp32 ulps of the weights
+    assert ((out[0] - ref).abs() <= ref.abs() * 2.0 ** -10.9 + 2.0 ** -24).all(), ((out[0] - ref) / ref).abs().max()
+
+
+@pytest.mark.parametrize("D,kv", [(96, BF), (256, BF), (128, F32)])
+def test_bf16_differences_of_weights(D, kv):
+    """Keys in pairs whose weights differ by 2^-13 / sqrt(D) of themselves and
+    whose V cancel but for that: the weights' last bits are the result."""
+    n, Hq = 128, 32
+    g = torch.Generator().manual_seed(D)
+    k = torch.randn(n // 2, 1, D, generator=g).to(BF).float().repeat_interleave(2, 0)
+    k[0::2, 0, 0], k[1::2, 0, 0] = 0.0, 1.0
+    q = torch.randn(1, Hq, D, generator=g).to(BF).float()
+    q[..., 0] = 2.0 ** -13
+    v = torch.ones(n, 1, D)
+    v[0::2] = -1.0
+    out = run(q, k, v, BF, kv)[0, :, 0].double()
+    s = (q[0].double() @ k[:, 0].double().t()) / math.sqrt(D)
+    ref = torch.softmax(s, -1) @ v[:, 0, 0].double()
+    rel = (out - ref) / ref
+    # bf16's rounding is at most 2^-9 of the result; an fp32 ulp of a score or a
+    # weight is up to ~2^-6 of a pair's difference, in either direction over 64 pairs
+    assert rel.square().mean().sqrt() < 0.01, rel

@@ -27,23 +27,16 @@ template <> __device__ __forceinline__ fp8e4m3 to_kv<fp8e4m3>(float x) { return 
 
 // 4 consecutive elements of one row, dims d .. d + 3: raw words in registers
 // until use, then the fp32 values the reference's gather gives (dims past D: 0).
+// V = 4 (D a multiple of 4): one load of all four, whatever the row's alignment
+// (global loads need none); a chunk past dim D re-reads the row's last one.
+// V = 2 (other D >= 4): the same, and last2 puts the dims of the chunk that
+// dim D cuts in place.  V = 1 (D < 4): element by element.
 template <typename KV> struct Raw4 { uint32_t w[sizeof(KV)]; };
-template <typename KV, bool VEC>
+template <typename KV, int V>
 __device__ __forceinline__ Raw4<KV> ld_raw4(const KV* row, int d, int D) {
   Raw4<KV> r;
-  if constexpr (VEC) {                           // D a multiple of 4, rows aligned to 4 elements
-    const KV* p = row + min(d, D - 4);
-    if constexpr (sizeof(KV) == 4) {
-      const u32x4 x = ld16(p);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) r.w[i] = x[i];
-    } else if constexpr (sizeof(KV) == 2) {
-      const u32x2 x = *reinterpret_cast<const u32x2*>(p);
-      r.w[0] = x[0];
-      r.w[1] = x[1];
-    } else {
-      r.w[0] = *reinterpret_cast<const uint32_t*>(p);
-    }
+  if constexpr (V > 1) {
+    __builtin_memcpy(&r, reinterpret_cast<const char*>(row + min(d, D - 4)), sizeof(r));
   } else {
 #pragma unroll
     for (int i = 0; i < (int)sizeof(KV); ++i) r.w[i] = 0u;
@@ -56,6 +49,16 @@ __device__ __forceinline__ Raw4<KV> ld_raw4(const KV* row, int d, int D) {
     }
   }
   return r;
+}
+// The chunk of dims D - 2, D - 1 (D even), loaded as the row's last four.
+template <typename KV>
+__device__ __forceinline__ void last2(Raw4<KV>& r, bool last) {
+  if constexpr (sizeof(KV) == 1) {
+    r.w[0] = last ? r.w[0] >> 16 : r.w[0];
+  } else {
+#pragma unroll
+    for (int i = 0; i < (int)sizeof(KV) / 2; ++i) r.w[i] = last ? r.w[i + sizeof(KV) / 2] : r.w[i];
+  }
 }
 template <typename KV, typename QT>
 __device__ __forceinline__ f32x4 widen4(const Raw4<KV>& r) {
@@ -114,6 +117,9 @@ __device__ __forceinline__ u32x2 pack4(const Raw4<KV>& r) {
 // instruction like an fp32 model's.  32 / 8 heads, us with P V in fp32 / three
 // parts (bf16): 1 x 2048 keys 48 / 43 at D = 96, 84 / 77 at 256; 64 x 2000 keys
 // 123 / 116 and 214 / 202; 2 x 300 rows 55 / 48 and 83 / 78.
+// Head dims that are no multiple of 4, and rows at odd offsets, read whole chunks
+// too: a 16-bit row of D = 50 loaded element by element into 256-dim registers took
+// 352 us (fp32 638) for one row on 2048 keys, 22 (37) so.
 // The waves' (max, sum, acc) merge through LDS at the end.  Latency-bound at
 // short contexts (one round trip per PF sub-tiles), HBM-bound beyond.  Against
 // one workgroup per (query head, query row) with VALU dot products, which read
@@ -128,22 +134,22 @@ __device__ __forceinline__ u32x2 pack4(const Raw4<KV>& r) {
 // workgroup of the first column stores them at their slots (block table); no
 // workgroup of the launch reads those slots.
 constexpr int kFusedRows = 16;
-template <typename KV, typename QT, int DP, bool VEC>
+template <typename KV, typename QT, int DP, int V>
 struct StreamCfg {
   static constexpr int kBytes = DP * (int)sizeof(KV);      // K (or V) bytes per key
-  static constexpr int kNW = kBytes > 512 || !VEC ? 4 : 8; // waves that split the keys (registers)
+  static constexpr int kNW = kBytes > 512 || V == 1 ? 4 : 8; // waves that split the keys (registers)
   static constexpr int kQS = DP + 4;                       // floats per LDS row of q, the new keys and the merge
   static constexpr int kMerge = kNW * 16 * kQS;
   template <bool FUSED> static constexpr int stage() { return (16 + (FUSED ? 32 : 0)) * kQS; }
   template <bool FUSED> static constexpr int lds() { return kMerge > stage<FUSED>() ? kMerge : stage<FUSED>(); }
-  // sub-tiles in flight beside the current one (registers; at DP 256 the eight
-  // waves overlap each other's loads instead; a 16-bit model's element loads
-  // leave no room for another one)
-  static constexpr int kPF = (DP == 256 && kNW == 8) || (!VEC && sizeof(QT) == 2) ? 0 : (VEC && kBytes <= 256 ? 2 : 1);
+  // sub-tiles in flight beside the current one (registers; at DP 256 the waves
+  // overlap each other's loads instead, and other head dims than multiples of
+  // 4 are rare)
+  static constexpr int kPF = V < 4 || DP == 256 ? 0 : (kBytes <= 256 ? 2 : 1);
 };
-template <bool DENSE, typename KV, typename QT, int DP, bool FUSED, bool VEC>
-__global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_stream_kernel(AttnArgs a) {
-  using Cfg = StreamCfg<KV, QT, DP, VEC>;
+template <bool DENSE, typename KV, typename QT, int DP, bool FUSED, int V>
+__global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_stream_kernel(AttnArgs a) {
+  using Cfg = StreamCfg<KV, QT, DP, V>;
   constexpr int NW = Cfg::kNW, PF = Cfg::kPF;
   constexpr int NT = DP / 16;             // K steps of 16 dims
   constexpr int NU = DP / 64;             // V column groups of 64 dims
@@ -222,7 +228,7 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
     }
     const KV* kp = kbase + row * kstride;
 #pragma unroll
-    for (int u = 0; u < NT; ++u) x.k[u] = ld_raw4<KV, VEC>(kp, 16 * u + 4 * grp, D);
+    for (int u = 0; u < NT; ++u) x.k[u] = ld_raw4<KV, V>(kp, 16 * u + 4 * grp, D);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {                // row of key 4grp + j: lane 4grp + j of the first 16 holds it
       const int src = 4 * grp + j;
@@ -230,7 +236,7 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
       const uint32_t hi = (uint32_t)__shfl((int)((uint64_t)row >> 32), src, 64);
       const KV* vp = vbase + (int64_t)(((uint64_t)hi << 32) | lo) * vstride;
 #pragma unroll
-      for (int u = 0; u < NU; ++u) x.v[j][u] = ld_raw4<KV, VEC>(vp, 64 * u + 4 * n, D);
+      for (int u = 0; u < NU; ++u) x.v[j][u] = ld_raw4<KV, V>(vp, 64 * u + 4 * n, D);
     }
     if constexpr (DENSE) {
 #pragma unroll
@@ -432,8 +438,16 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
     }
   };
   const bool tail = D != DP;
-  auto compute = [&](int t, const Tile& x) {
+  auto compute = [&](int t, Tile& x) {
     const int p0 = 16 * (wave + NW * t);
+    if constexpr (V == 2) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) last2(x.k[u], 16 * u + 4 * grp + 2 == D);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) last2(x.v[j][u], 64 * u + 4 * n + 2 == D);
+    }
     const int lim = min(vis, nkeys - 1) - p0;
     const bool mask = p0 + 16 > nkeys || (!DENSE && p0 + 15 > ctx);
     if constexpr (k16) {
@@ -540,16 +554,19 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, VEC>::kNW)) attn_s
 
 template <bool DENSE, typename KV, typename QT, bool FUSED>
 static hipError_t launch_stream_d(const AttnArgs& a, dim3 grid, hipStream_t st) {
-  auto go = [&](auto dp, auto vec) {
-    constexpr int DP = decltype(dp)::value;
-    constexpr bool VEC = decltype(vec)::value;
-    const dim3 block(64 * StreamCfg<KV, QT, DP, VEC>::kNW);
-    hipLaunchKernelGGL((attn_stream_kernel<DENSE, KV, QT, DP, FUSED, VEC>), grid, block, 0, st, a);
+  auto go = [&](auto dp, auto v) {
+    constexpr int DP = decltype(dp)::value, V = decltype(v)::value;
+    const dim3 block(64 * StreamCfg<KV, QT, DP, V>::kNW);
+    hipLaunchKernelGGL((attn_stream_kernel<DENSE, KV, QT, DP, FUSED, V>), grid, block, 0, st, a);
   };
-  if (!a.vec_rows) go(std::integral_constant<int, 256>(), std::false_type());   // rare: odd alignment or head dim
-  else if (a.head_dim <= 64) go(std::integral_constant<int, 64>(), std::true_type());
-  else if (a.head_dim <= 128) go(std::integral_constant<int, 128>(), std::true_type());
-  else go(std::integral_constant<int, 256>(), std::true_type());
+  auto by_dim = [&](auto v) {
+    if (a.head_dim <= 64) go(std::integral_constant<int, 64>(), v);
+    else if (a.head_dim <= 128) go(std::integral_constant<int, 128>(), v);
+    else go(std::integral_constant<int, 256>(), v);
+  };
+  if (a.head_dim % 4 == 0) by_dim(std::integral_constant<int, 4>());
+  else if (a.head_dim > 4) by_dim(std::integral_constant<int, 2>());
+  else go(std::integral_constant<int, 64>(), std::integral_constant<int, 1>());
   return hipGetLastError();
 }
 

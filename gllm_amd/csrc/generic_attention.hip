@@ -23,14 +23,15 @@ hipError_t launch_generic_f16(const AttnArgs& a, bool tile, bool dense, dim3 gri
 
 static hipError_t launch_kind(AttnArgs a, bool tile, bool dense, dim3 grid, hipStream_t st) {
   const size_t eq = a.dtype == kF32 ? 4 : 2;
-  const size_t ek = dense ? eq : (a.kv_dtype == kF32 ? 4 : (a.kv_dtype == kFP8 ? 1 : 2));
-  const size_t al = tile ? 16 : 4 * ek;           // bytes of one K/V load
-  const auto rows = [&](const void* p, int64_t stride, int64_t batch) {
-    return ((uintptr_t)p & (al - 1)) == 0 && (size_t)stride * ek % al == 0 && (size_t)batch * ek % al == 0;
-  };
-  a.vec_rows = (size_t)a.head_dim * ek % al == 0 &&
-               (dense ? rows(a.k, a.k_row_stride, a.k_batch_stride) && rows(a.v, a.v_row_stride, a.v_batch_stride)
-                      : rows(a.k_cache, a.cache_slot_stride, 0) && rows(a.v_cache, a.cache_slot_stride, 0));
+  if (tile) {                                      // 16-byte chunks of K/V
+    const size_t ek = dense ? eq : (a.kv_dtype == kF32 ? 4 : (a.kv_dtype == kFP8 ? 1 : 2));
+    const auto rows = [&](const void* p, int64_t stride, int64_t batch) {
+      return ((uintptr_t)p & 15) == 0 && (size_t)stride * ek % 16 == 0 && (size_t)batch * ek % 16 == 0;
+    };
+    a.vec_rows = (size_t)a.head_dim * ek % 16 == 0 &&
+                 (dense ? rows(a.k, a.k_row_stride, a.k_batch_stride) && rows(a.v, a.v_row_stride, a.v_batch_stride)
+                        : rows(a.k_cache, a.cache_slot_stride, 0) && rows(a.v_cache, a.cache_slot_stride, 0));
+  }
   a.vec_out = a.head_dim % 4 == 0 && a.out_row_stride % 4 == 0 && ((uintptr_t)a.out & (4 * eq - 1)) == 0;
   switch (a.dtype) {
     case kF32: return launch_generic_f32(a, tile, dense, grid, st);

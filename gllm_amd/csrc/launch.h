@@ -121,7 +121,7 @@ struct AttnArgs {
   const WorkItem* tile_items;  // the tiled kernel's work (null: a grid over every sequence)
   int32_t n_tile_items;
   int32_t tile_min_q;
-  int32_t vec_rows;            // K/V rows aligned for the kernel's vector loads (set by the launcher)
+  int32_t vec_rows;            // tiled kernel: K/V rows in whole aligned 16-byte chunks (set by the launcher)
   int32_t vec_out;             // output rows aligned for stores of 4 elements (set by the launcher)
 };
 

@@ -60,6 +60,29 @@ def test_paged_unaligned_rows():
         _check(out, oracle_paged(b), "unaligned")
 
 
+@pytest.mark.parametrize("dtype,kv,D,off", [
+    (F32, F32, 2, 0), (BF, BF, 2, 1), (BF, BF, 50, 0), (BF, torch.float8_e4m3fn, 34, 3), (F16, F16, 126, 0),
+    (BF, BF, 130, 1), (F16, F32, 250, 0), (F32, F32, 254, 1), (F16, F16, 96, 1), (BF, F32, 64, 1)])
+def test_paged_odd_head_dims_and_rows(dtype, kv, D, off):
+    """Head dims that are no multiple of 4 and rows at odd offsets: the last row
+    of the pool ends where its buffer does, so a load past a row's end would be
+    past the buffer's."""
+    for ctx, ql in (FEW, MANY):
+        b = make_batch(ctx, ql, 16, 4, D, dtype=dtype)
+        ns, row = b.k_cache.shape[0], 4 * D
+        caches = []
+        for c in (b.k_cache, b.v_cache):
+            buf = torch.zeros(ns * (row + off) + off, device=DEV).to(kv)
+            view = buf[off:].unflatten(0, (ns, row + off))[:, :row].unflatten(1, (4, D))
+            view.copy_(c.to(kv))
+            caches.append(view)
+        plan = paged.AttentionPlan(b.q_lens, b.seq_lens, num_q_heads=16, num_kv_heads=4, head_dim=D, block_size=16,
+                                   dtype=dtype, device=DEV)
+        out = paged.paged_attention(plan, b.q, caches[0], caches[1], b.block_table)
+        b.k_cache, b.v_cache = (c.contiguous().to(dtype) for c in caches)
+        _check(out, oracle_paged(b), f"{dtype} {kv} {D} +{off}")
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("B,Tq,T,Hq,Hkv,D", [(1, 5, 33, 8, 2, 48), (2, 40, 65, 8, 2, 80), (3, 300, 333, 32, 8, 96)])
 def test_dense_masks(dtype, B, Tq, T, Hq, Hkv, D):

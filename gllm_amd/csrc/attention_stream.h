@@ -345,7 +345,9 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
   // 64u + 4n .. + 3 of key 4grp + j (fp32 values, or packed words of a 16-bit
   // model); lim: keys 4grp + j <= lim are visible
   auto tile = [&](auto kf, auto vf, int lim, bool mask, const float* bias) {
-    f32x4 s = {0.f, 0.f, 0.f, 0.f}, s1 = s;      // two chains: half the length of the fp32 sums
+    // two chains: half the length of the fp32 sums; from 128 dims on, the fp32
+    // products' in two halves of the dims
+    f32x4 s = {0.f, 0.f, 0.f, 0.f}, s1 = s, sh = s;
     if constexpr (k16) {
 #pragma unroll
       for (int u = 0; u < NT / 2; ++u) {
@@ -356,6 +358,10 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
     } else {
 #pragma unroll
       for (int u = 0; u < NT; ++u) {
+        if (DP >= 128 && u == NT / 2) {
+          sh = s + s1;
+          s = s1 = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
         const f32x4 kk = kf(u);
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
@@ -365,6 +371,7 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
       }
     }
     s += s1;
+    if (!k16 && DP >= 128) s += sh;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       s[j] *= a.scale;

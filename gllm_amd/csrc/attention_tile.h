@@ -245,11 +245,14 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
           bv[j] = (float)brow[min(p, TK - 1)];
         }
       }
-      f32x16 s, s1;                                // two chains: half the length of the fp32 sums
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[j] = s1[j] = 0.f;
+      // two chains: half the length of the fp32 sums; at 256 dims in two halves
+      f32x16 s = f32x16{}, s1 = f32x16{}, sh = f32x16{};
 #pragma unroll
       for (int u = 0; u < DP / 8; ++u) {
+        if (DP == 256 && u == DP / 16) {
+          sh = s + s1;
+          s = s1 = f32x16{};
+        }
         const f32x4 kv4 = *reinterpret_cast<const f32x4*>(&lds[b][0][n][8 * u + 4 * h]);
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
@@ -257,8 +260,8 @@ __global__ void __launch_bounds__(256) attn_tile_kernel(AttnArgs a) {
           s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(kv4[e + 1], qv[u][e + 1], s1, 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[j] += s1[j];
+      s += s1;
+      if (DP == 256) s += sh;
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         s[j] *= a.scale;

@@ -5,6 +5,7 @@ import math
 import pytest
 import torch
 
+import gllm_amd
 from gllm_amd import paged
 
 pytestmark = pytest.mark.gpu
@@ -73,3 +74,22 @@ def test_bf16_differences_of_weights(D, kv):
     # bf16's rounding is at most 2^-9 of the result; an fp32 ulp of a score or a
     # weight is up to ~2^-6 of a pair's difference, in either direction over 64 pairs
     assert rel.square().mean().sqrt() < 0.01, rel
+
+
+@pytest.mark.parametrize("B,Tq,D,part", [(1, 1, 64, 2), (1, 1, 128, 4), (1, 1, 256, 4), (3, 300, 256, 4)])
+def test_f32_score_sums_are_short(B, Tq, D, part):
+    """Key 0's score is 256 plus D - 4 products of 2^-17, each lost when it is added
+    to the 256 (half an ulp is 2^-16); key 1's is the exact sum.  The result, (p0 - p1)
+    / (p0 + p1), shows how many met the 256: the dims of one partial sum, D / part."""
+    n = D - 4
+    q, k = torch.zeros(B, Tq, 32, D), torch.zeros(B, 2, 8, D)
+    q[..., 0], q[..., 1:n + 1] = 16.0, 2.0 ** -8
+    k[:, 0, :, 0], k[:, 0, :, 1:n + 1] = 16.0, 2.0 ** -9
+    k[:, 1, :, 0] = 16.0 + n * 2.0 ** -21              # a multiple of fp32's 2^-19 there
+    v = torch.ones(B, 2, 8, D)
+    v[:, 1] = -1.0
+    out = gllm_amd.reference_attention(q.to(DEV), k.to(DEV), v.to(DEV), torch.zeros(B, Tq, 2, device=DEV)).cpu()
+    lost = out.double().abs() * 2 * math.sqrt(D) * 2.0 ** 17   # s1 - s0 = lost 2^-17 / sqrt(D); tanh(x / 2) = x / 2 here
+    # an ulp of a scaled score (2^-20 at 16, 2^-19 at 32) is 2 of these at most, and
+    # each of the two scores is rounded once; the weights' ulps are a tenth of that
+    assert lost.max() <= D / part + 4, lost.max()

@@ -111,12 +111,10 @@ __device__ __forceinline__ u32x2 pack4(const Raw4<KV>& r) {
 //     already the B operand of step j; A is V[key 4grp + j][64u + 4n + e], so
 //     one 4-element load per (j, u) feeds the four output blocks e.
 // A 16-bit model's K, V and q are 16-bit values, so its S runs on the 16x16x32
-// instruction (products exact, fp32 sums).  P stays an fp32 value: in bf16, whose
-// exponents are fp32's, as the sum of three parts (24 bits) on 16x16x16; fp16
-// parts of a small p would be subnormal, so an fp16 model's P V runs on the fp32
-// instruction like an fp32 model's.  32 / 8 heads, us with P V in fp32 / three
-// parts (bf16): 1 x 2048 keys 48 / 43 at D = 96, 84 / 77 at 256; 64 x 2000 keys
-// 123 / 116 and 214 / 202; 2 x 300 rows 55 / 48 and 83 / 78.
+// instruction (products exact, fp32 sums).  P stays in fp32, and so does P V: P in
+// two 16-bit parts lost bits (fp16 parts of a small p are subnormal) and turned an
+// infinity in V into a NaN, and three parts with V's infinities kept from the low
+// ones cost as much as fp32 (bf16, 1 x 2048 keys, D = 96 and 256: 48 and 86 us).
 // Head dims that are no multiple of 4, and rows at odd offsets, read whole chunks
 // too: a 16-bit row of D = 50 loaded element by element into 256-dim registers took
 // 352 us (fp32 638) for one row on 2048 keys, 22 (37) so.
@@ -155,7 +153,6 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
   constexpr int NU = DP / 64;             // V column groups of 64 dims
   constexpr int QS = Cfg::kQS;
   constexpr bool k16 = sizeof(QT) == 2;   // 16-bit MFMA (above)
-  constexpr bool kSplitP = std::is_same<QT, __bf16>::value;   // p in three parts (above)
   // q of the columns, the new keys' K and V (FUSED); the merge reuses the area
   __shared__ __attribute__((aligned(16))) float lds[Cfg::template lds<FUSED>()];
   __shared__ float mml[NW][16][2];
@@ -279,8 +276,12 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
   if constexpr (FUSED) {
     // element pairs (token t, dims j and j + D/2)
     const bool writer = wgrp == 0;
-    for (int e = tid; e < qlen * (DP / 2); e += 64 * NW) {
+    for (int e = tid; e < 16 * (DP / 2); e += 64 * NW) {
       const int t = e / (DP / 2), j = e - t * (DP / 2);
+      if (t >= qlen) {                             // no such key: weight 0, V 0
+        nv[t][2 * j] = nv[t][2 * j + 1] = 0.f;
+        continue;
+      }
       if (j >= half) {
         nk[t][2 * j] = nk[t][2 * j + 1] = 0.f;
         nv[t][2 * j] = nv[t][2 * j + 1] = 0.f;
@@ -388,60 +389,27 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
     l = l * alpha + ((s[0] + s[1]) + (s[2] + s[3]));
     m = mn;
     // the sub-tile's P V from zero, then one FMA per output with the rescale
-    auto rescale = [&](int u, int e, const f32x4& w) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o[u][e][i] = __builtin_fmaf(o[u][e][i], alpha, w[i]);
-    };
-    if constexpr (kSplitP) {
-      // p = p0 + p1 + p2 in bf16: 24 bits, the low parts added first
-      u32x2 pp[3];
-      f32x4 r = s;
+    for (int u = 0; u < NU; ++u) {
+      f32x4 w[4];
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        pp[c] = u32x2{E16<QT>::pack2(r[0], r[1]), E16<QT>::pack2(r[2], r[3])};
+      for (int e = 0; e < 4; ++e) w[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          r[2 * i] -= E16<QT>::lo(pp[c][i]);
-          r[2 * i + 1] -= E16<QT>::hi(pp[c][i]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        u32x2 vv[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) vv[j] = vf(j, u);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {   // element e of the four keys: halves of word e / 2
-          const uint32_t sel = e % 2 ? 0x07060302u : 0x05040100u;
-          const u32x2 av = {__builtin_amdgcn_perm(vv[1][e / 2], vv[0][e / 2], sel),
-                            __builtin_amdgcn_perm(vv[3][e / 2], vv[2][e / 2], sel)};
-          f32x4 w = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int c = 2; c >= 0; --c) w = E16<QT>::mfma16k16(av, pp[c], w);
-          rescale(u, e, w);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        f32x4 w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          f32x4 vv;
-          if constexpr (k16) {
-            const u32x2 x = vf(j, u);
-            vv = f32x4{E16<QT>::lo(x[0]), E16<QT>::hi(x[0]), E16<QT>::lo(x[1]), E16<QT>::hi(x[1])};
-          } else {
-            vv = vf(j, u);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[j], w[e], 0, 0, 0);
+      for (int j = 0; j < 4; ++j) {
+        f32x4 vv;
+        if constexpr (k16) {
+          const u32x2 x = vf(j, u);
+          vv = f32x4{E16<QT>::lo(x[0]), E16<QT>::hi(x[0]), E16<QT>::lo(x[1]), E16<QT>::hi(x[1])};
+        } else {
+          vv = vf(j, u);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) rescale(u, e, w[e]);
+        for (int e = 0; e < 4; ++e) w[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[j], w[e], 0, 0, 0);
       }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[u][e][i] = __builtin_fmaf(o[u][e][i], alpha, w[e][i]);
     }
   };
   const bool tail = D != DP;
@@ -509,7 +477,7 @@ __global__ void __launch_bounds__((64 * StreamCfg<KV, QT, DP, V>::kNW)) attn_str
         else return x;
       };
       tile([&](int u) { return get(&nk[min(n, qlen - 1)][16 * u + 4 * grp]); },
-           [&](int j, int u) { return get(&nv[min(4 * grp + j, qlen - 1)][64 * u + 4 * n]); }, r, true, nullptr);
+           [&](int j, int u) { return get(&nv[4 * grp + j][64 * u + 4 * n]); }, r, true, nullptr);
     }
   }
   l = sum_xor32(sum_xor16(l));

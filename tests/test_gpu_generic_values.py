@@ -76,6 +76,35 @@ def test_bf16_differences_of_weights(D, kv):
     assert rel.square().mean().sqrt() < 0.01, rel
 
 
+@pytest.mark.parametrize("dtype,kv,D", [(BF, BF, 96), (BF, F32, 64), (F16, F16, 256), (F32, F32, 64), (BF, BF, 50)])
+@pytest.mark.parametrize("rows,n,fused", [(1, 64, False), (3, 80, False), (200, 256, False),
+                                          (1, 37, True), (3, 50, True), (16, 64, True)])
+def test_infinities_in_v(dtype, kv, D, rows, n, fused):
+    """An infinity in V at a key that every row sees is the result in its dim, as
+    weight times infinity is for any weight above 0: at the first key, at the one
+    that takes the largest weight and at the last row's own key, also where that is
+    the new token which the launch writes, whatever the number of keys."""
+    g = torch.Generator().manual_seed(n)
+    Hq, Hkv = 64, 16                                 # tiled from ~190 rows on
+    q = torch.randn(rows, Hq, D, generator=g)
+    k, v = torch.randn(n, Hkv, D, generator=g), torch.randn(n, Hkv, D, generator=g)
+    top = n - rows                                   # the newest key that every row sees
+    k[5] *= 4.0 / math.sqrt(D)
+    k[5, :, 0] += 3.0
+    q[..., 0] += 3.0
+    v[0, :, 1], v[5, :, 2], v[top, :, 3], v[n - 1, :, 4] = math.inf, -math.inf, math.inf, -math.inf
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    if not fused:
+        out = run(q, k, v, dtype, kv)
+    else:                                            # the new rows' keys come with the call
+        kc, vc = k.clone(), v.clone()
+        kc[n - rows:], vc[n - rows:] = 0.0, 0.0
+        out = run(q, kc, vc, dtype, kv, kv_new=(k[n - rows:], v[n - rows:]))
+    assert (out[..., 1] == math.inf).all() and (out[..., 2] == -math.inf).all() and (out[..., 3] == math.inf).all()
+    assert (out[-1, :, 4] == -math.inf).all()        # the earlier rows give it weight 0: NaN, as in the reference
+    assert torch.isfinite(out[..., 5:].float()).all() and torch.isfinite(out[..., 0].float()).all()
+
+
 @pytest.mark.parametrize("B,Tq,D,part", [(1, 1, 64, 2), (1, 1, 128, 4), (1, 1, 256, 4), (3, 300, 256, 4)])
 def test_f32_score_sums_are_short(B, Tq, D, part):
     """Key 0's score is 256 plus D - 4 products of 2^-17, each lost when it is added

@@ -1015,11 +1015,13 @@ struct QKVTiles { int64_t full, half; double rounds; };
 static QKVTiles qkv_tiles(int64_t n, int ngroups, int cus) {
   const int64_t halves = (n + 127) / 128;
   QKVTiles best{0, 0, 0.0};
-  // as many full tiles as whole rounds hold, one round fewer, or all of them
+  // as many full tiles as whole rounds hold, one round fewer, all of them, or as
+  // many as fill the last round of full tiles short of its end (9 of 28 column
+  // groups on 256 CUs: 252 workgroups; 2,500 tokens of hidden 5120 248 us without)
   const int64_t per = std::max<int64_t>(1, cus / ngroups), all = (n + 255) / 256, fit = n / 256;
-  const int64_t r = std::min(fit * ngroups / cus, fit / per + 1);
-  for (int64_t c = 0; c < 3; ++c) {
-    const int64_t full = c == 2 ? all : std::max<int64_t>(0, std::min(fit, (r - c) * cus / ngroups));
+  const int64_t r = std::min(fit * ngroups / cus, fit / per + 1), last = (fit * ngroups + cus - 1) / cus;
+  for (int64_t c = 0; c < 4; ++c) {
+    const int64_t full = c == 2 ? all : std::max<int64_t>(0, std::min(fit, (c == 3 ? last : r - c) * cus / ngroups));
     const int64_t half = c == 2 ? 0 : halves - 2 * full;
     const int64_t fw = full * ngroups, hw = half * ngroups;
     const int64_t fr = (fw + cus - 1) / cus, spare = fr * cus - fw;   // half tiles start in the full ones' last round

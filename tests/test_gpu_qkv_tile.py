@@ -48,3 +48,9 @@ def test_tile256_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad):
     kc[slots[ok]], vc[slots[ok]] = k[ok].to(kv), v[ok].to(kv)
     assert torch.equal(_bits(qd)[real], _bits(q)[real]) and (qd.cpu()[~real] == 9.0).all()
     assert torch.equal(_bits(kd), _bits(kc)) and torch.equal(_bits(vd), _bits(vc))
+
+
+@pytest.mark.parametrize("n,hidden,Hq,Hkv,D,kv,rot,pad", [
+    (2500, 64, 40, 8, 128, BF, True, False)])   # 9 full tiles: the last round of full tiles ends short
+def test_short_last_round_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad):
+    test_tile256_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad)

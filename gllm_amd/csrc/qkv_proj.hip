@@ -1126,10 +1126,23 @@ hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
       (!a.q_out || (al16(a.q_out) && a.q_out_row_stride % 8 == 0))) {
     const int ngroups = heads / hp;
     const QKVTiles t = qkv_tiles(a.num_tokens, ngroups, a.cus);
-    // below 2 / 5 of the CUs the 128-token x one-head tiles spread the work wider
-    // (1B layer, us, these / those: 1024 tokens, 96 workgroups, 33.0 / 29.8; 1536,
-    // 144 workgroups, 33.8 / 51.2; 8B 700 tokens, 144 workgroups, 60.5 / 71.0)
-    if (5 * (t.full + t.half) * ngroups >= 2 * a.cus) {
+    // The 128-token x one-head tiles keep a batch that they finish in one go, two per
+    // CU on the fullest XCD (super-groups are dealt out whole): always at head dim 64,
+    // at 128 unless they are so many per CU that their starts weigh more: over 1 up to
+    // hidden 2560, from 1.5 at 4096-4608; between and above they stay ahead or even.
+    // Measured over 20 layers, 300-3,071 tokens (us, those / these): head dim 64: 48 heads,
+    // hidden 2048, 1,024 tokens 29 / 33; 64 heads, 3072, 1,024 / 1,100 (not one go) 45 / 62,
+    // 72 / 60.  Head dim 128: 32 heads, 2048, 1,024 / 1,100 (1.0, 1.1 per CU) 32 / 34, 41 / 34;
+    // 28 heads, 2560, 1,300 (1.2) 49 / 42; 40 heads, 3072, 900 / 1,300 / 1,536 (1.25, 1.7, 1.9)
+    // 58 / 62, 59 / 62, 66 / 64; 40 heads, 4096, 1,300 (1.7) 79 / 73; 48 heads, 4096, 700 / 900 /
+    // 1,300 (1.1, 1.5, not one go) 71 / 73, 80 / 73, 118 / 96; 56 heads, 5120, 700 / 1,024
+    // (1.3, 1.75) 86 / 103, 98 / 106; 64 heads, 6144, 700 / 1,024 (1.5, 2.0) 101 / 119, 115 / 117;
+    // 80 heads, 8192, 512 / 700 (1.25, not one go) 145 / 153, 230 / 152.
+    const QKVGroups gr = qkv_groups(tiles, heads, a.cus);
+    const bool one_go = (gr.nsg + kXcds - 1) / kXcds * gr.gt * gr.gh <= 2 * (int64_t)a.cus / kXcds;
+    const int64_t small = tiles * heads;
+    const bool ahead = a.hidden <= 2560 ? small > a.cus : a.hidden >= 4096 && a.hidden <= 4608 && 2 * small >= 3 * a.cus;
+    if (!one_go || (a.head_dim == 128 && ahead)) {
       const auto wgs_of = [&](int64_t tiles) { return (tiles * ngroups + kXcds - 1) / kXcds * kXcds; };
       b.full_tiles = (int32_t)t.full;
       b.half_tiles = (int32_t)t.half;

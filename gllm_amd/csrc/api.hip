@@ -179,6 +179,7 @@ struct gllm_attn_plan {
   int32_t num_seqs = 0, Hq = 0, Hkv = 0, D = 0, bs = 0, dtype = 0;
   int32_t split_len = 0, max_q = 0;
   int32_t n_decode_seqs = 0, n_prefill_seqs = 0, heads_per_wg = 8, decode_waves = 8, prefill_waves = 8;
+  bool prefill_pairs = false;  // prefill-only launches at D = 64: two workgroups per CU
   bool mfma = false;      // bf16 head dim 64 / 128: the MFMA kernels; otherwise the generic kernel
   int64_t total_rows = 0;
   int64_t n_partials = 0;
@@ -837,6 +838,25 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
       for (const PrefillPiece& pc : pcs) pf.push_back({pc.kend, pc.it});
     }
     longest_first(pf);
+    // Two prefill workgroups per CU (D = 64) run a start under the other's keys, but
+    // spill: they pay where items are many and short (from two per CU, 320 keys on
+    // average), or at eight and more per CU without cached context.  Measured, bf16,
+    // 32 / 8 heads (us, one / two per CU; items, keys an item): 16 x 256 tokens 21.0 / 20.4
+    // (512, 160), 32 x 256 48.3 / 39.5 (1,024, 160), 64 x 256 81.1 / 71.4 (2,048, 160), 24 x 384
+    // 48.7 / 46.7 (1,152, 224), 16 x 1,024 123.5 / 118.6 (2,048, 528), 8 of 512-4,096 303 / 296;
+    // the other side: 1 x 2,048 44.5 / 52.0 (256), 4 x 1,024 33.1 / 37.9 (512, 528), 2 x 4,096
+    // 173 / 177 (1,024), 64 x 64 on 1,000 65.7 / 64.8, 109 x 132 on 1,024 279 / 303 (2,616, 1,132),
+    // 32 x 1,024 256 / 258.  fp16 and an fp8 cache lose 2-45% everywhere and stay at one.
+    if (!pf.empty() && head_dim == 64) {
+      int64_t keys = 0;
+      bool context = false;
+      for (const Keyed& k : pf) {
+        keys += k.work;
+        context = context || k.it.ctx_len > 0;
+      }
+      const int64_t n = (int64_t)pf.size();
+      p->prefill_pairs = (n >= 2 * (int64_t)cus && keys <= 320 * n) || (n >= 8 * (int64_t)cus && !context);
+    }
     // A decode-only batch of fewer than two items per CU whose items leave the
     // CUs unevenly loaded goes page-balanced: its partials and their merge cost
     // ~8 us, which a CU streams 256 KB in.  Measured (split / page-balanced us,
@@ -1101,6 +1121,7 @@ static int paged_attention_impl(const gllm_attn_plan* p, const void* q, int64_t 
   a.heads_per_wg = p->heads_per_wg;
   a.decode_waves = p->decode_waves;
   a.prefill_waves = p->prefill_waves;
+  a.prefill_pairs = p->prefill_pairs;
   // the MFMA kernels read a cache in the model dtype or fp8; a 16-bit model
   // over an f32 (or the other 16-bit) cache takes the generic kernel, which
   // rounds each cached value to the model dtype as the reference's gather does

@@ -1256,11 +1256,11 @@ __global__ void __launch_bounds__(64 * kWaves) mixed_balanced_kernel(AttnArgs a)
 }
 
 // Prefill items only: kPrefillOnlyWaves-wave workgroups with a
-// kPrefillOnlyStages-stage ring.  D = 64: two workgroups per CU (128 registers,
-// 69 KB of LDS each), so one's start and barriers run under the other: 8
-// prompts of 512-4096 tokens, 32 / 8 heads, 328 -> 315 us.
-template <typename T, int D, bool KV8>
-__global__ void __launch_bounds__(64 * kPrefillOnlyWaves) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2)))
+// kPrefillOnlyStages-stage ring.  PAIR (bf16, D = 64, 16-bit cache): two
+// workgroups per CU (128 registers, some of them in scratch, 69 KB of LDS each),
+// so one's start and barriers run under the other; the plan says when that pays.
+template <typename T, int D, bool KV8, bool PAIR = false>
+__global__ void __launch_bounds__(64 * kPrefillOnlyWaves) __attribute__((amdgpu_waves_per_eu(PAIR ? 4 : 2)))
 prefill_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) char lds[PrefillCfg<D, kPrefillOnlyStages>::kLdsBytes];
   const WorkItem it = a.items[blockIdx.x];
@@ -1285,6 +1285,12 @@ static void launch_paged_hk(const AttnArgs& a, bool pf, bool dc, hipStream_t st)
     if constexpr (HW * KW == kWaves)
       hipLaunchKernelGGL((paged_attn_kernel<T, D, true, true, HW, KW, KV8>), grid, dim3(64 * kWaves), 0, st, a);
   } else if (pf) {
+    if constexpr (std::is_same_v<T, __bf16> && D == 64 && !KV8) {
+      if (a.prefill_pairs) {
+        hipLaunchKernelGGL((prefill_kernel<T, D, KV8, true>), grid, dim3(64 * kPrefillOnlyWaves), 0, st, a);
+        return;
+      }
+    }
     hipLaunchKernelGGL((prefill_kernel<T, D, KV8>), grid, dim3(64 * kPrefillOnlyWaves), 0, st, a);
   } else {
     hipLaunchKernelGGL((paged_attn_kernel<T, D, false, true, HW, KW, KV8>), grid, dim3(64 * HW * KW), 0, st, a);

@@ -46,6 +46,17 @@ def _layer(B, Tq, Hq, Hkv, D, dtype, kv, odd=False):
     return gllm_amd.Attention(0, Cfg, w), x, ang.cos().to(dtype).to(DEV), ang.sin().to(dtype).to(DEV), pool, meta
 
 
+def _routes(att):
+    """What each call of forward's fused route returned."""
+    seen, fused = [], att._fused_decode
+
+    def spy(*args):
+        seen.append(fused(*args))
+        return seen[-1]
+    att._fused_decode = spy
+    return seen
+
+
 def _by_linear(att, x, cos, sin, pool, meta):
     B, Tq, _ = x.shape
     q, k, v = (F.linear(x, w).view(B, Tq, -1, att.head_dim) for w in (att.W_q, att.W_k, att.W_v))
@@ -57,7 +68,9 @@ def _by_linear(att, x, cos, sin, pool, meta):
 def test_fused_decode(B, Tq, Hq, Hkv, D, kv):
     att, x, cos, sin, pool, meta = _layer(B, Tq, Hq, Hkv, D, BF, kv)
     p1, p2 = pool.clone(), pool.clone()
+    seen = _routes(att)
     out, ref = att.forward(x, cos, sin, p1, meta), _by_linear(att, x, cos, sin, p2, meta)
+    assert len(seen) == 1 and seen[0] is not None
     assert_close_bf16(out, ref, "forward")
     # the written rows: projections summed in another order, so a step of the
     # cache dtype on few values (bf16 2^-7 after the rotation's roundings, fp8 2^-3)
@@ -71,5 +84,7 @@ def test_fused_decode(B, Tq, Hq, Hkv, D, kv):
 def test_other_calls_keep_their_route(dtype, odd):
     att, x, cos, sin, pool, meta = _layer(9, 1, 8, 2, 64, dtype, dtype, odd)
     p1, p2 = pool.clone(), pool.clone()
+    seen = _routes(att)
     assert torch.equal(att.forward(x, cos, sin, p1, meta), _by_linear(att, x, cos, sin, p2, meta))
     assert torch.equal(p1, p2)
+    assert seen in ([], [None])

@@ -127,7 +127,7 @@ def test_config_c_prefill_full():
 @pytest.mark.parametrize("split", [0, paged.BALANCED])
 def test_config_d_mixed_full(split):
     """Config (d) in one launch: the item plan, and the page-balanced decode
-    share with prefill items (twice: the split tickets are re-armed)."""
+    share with prefill items (twice, over the same workspace)."""
     print(f"config d full split={split}", flush=True)
     b = workloads.materialize(workloads.config_d(), DEV, values_on_device=True)
     plan = _plan(b, split_tokens=split)

@@ -103,7 +103,7 @@ def test_decode_parity(Hq, Hkv, D, split):
     plan = paged.AttentionPlan(b.q_lens, b.seq_lens, num_q_heads=Hq, num_kv_heads=Hkv, head_dim=D,
                                block_size=16, dtype=torch.bfloat16, device=DEV, split_tokens=split)
     ref = oracle_paged(b)
-    for rep in range(2):  # second launch checks the split tickets were reset
+    for rep in range(2):  # the second launch finds the first one's partials in its workspace
         out = paged.paged_attention(plan, b.q, b.k_cache, b.v_cache, b.block_table)
         torch.cuda.synchronize()
         assert_close_bf16(out, ref, f"decode rep {rep}")
@@ -265,7 +265,7 @@ def test_mixed_batch_one_launch(split):
     assert info["decode_seqs"] == 3 and info["prefill_seqs"] == 3
     assert (info["decode_segments"] > 0) == (split == paged.BALANCED)
     ref = oracle_paged(b)
-    for rep in range(2):   # the second launch finds the split tickets re-armed
+    for rep in range(2):   # the second launch finds the first one's partials in its workspace
         out = paged.paged_attention(plan, b.q, b.k_cache, b.v_cache, b.block_table)
         torch.cuda.synchronize()
         assert_close_bf16(out, ref, f"mixed rep {rep}")

@@ -343,15 +343,18 @@ def test_qkv_random_shapes_exact(n, hidden, Hq, Hkv, D, kvd, rotate_q, with_q):
 
 
 @pytest.mark.parametrize("integer,rotate_q", [(True, True), (False, True), (True, False)])
-def test_qkv_large_batch_unfused_route(integer, rotate_q):
-    """From paged.QKV_UNFUSED_FROM tokens the projections go through F.linear
+def test_qkv_large_batch_unfused_route(integer, rotate_q, monkeypatch):
+    """From the token count a caller names the projections go through F.linear
     (hipBLASLt) and then the RoPE + KV write kernel: same results as the
     oracle (exact on small-integer data, within the GEMM's rounding on N(0,1)
     data), untouched slots keep their sentinel."""
     n = paged.QKV_UNFUSED_FROM + 300
     print(f"qkv unfused route n={n} integer={integer} rotate_q={rotate_q}", flush=True)
+    calls, linear = [], paged.F.linear
+    monkeypatch.setattr(paged.F, "linear", lambda *args: calls.append(args[0].is_cuda) or linear(*args))
     q, qr, kc, vc, kr, vr, slots, ns = _run(n, 256, 8, 2, 128, integer, 41, rotate_q=rotate_q,
                                             unfused_from=paged.QKV_UNFUSED_FROM)
+    assert sum(calls) == 3
     if integer:
         assert torch.equal(q.cpu().view(torch.int16), qr.view(torch.int16))
         assert torch.equal(kc.view(torch.int16), kr.view(torch.int16))

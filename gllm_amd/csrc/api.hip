@@ -863,7 +863,11 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     // 8B heads; longest CU's excess over the mean): 48 sequences of 1100 keys
     // 57.4 / 50.3 (excess 275 KB), 32 of 500-3000 65.6 / 49.7 (660 KB), 40 of
     // 4000 161 / 121 (1.5 MB); 90 of 500-2000 92.3 / 94.5 (190 KB), 160 of
-    // 300-900 84.1 / 85.7 (210 KB).  In a mixed launch, where the prefill items
+    // 300-900 84.1 / 85.7 (210 KB), 96 of 128-2048 92.4 / 94.7; with an fp8 cache, whose
+    // bytes the plan does not know (it counts 16-bit ones), 40 of 1100 34.4 / 28.2, 80 of
+    // 128-2048 48.0 / 43.2, 96 53.1 / 54.6.  Head dim 64, 32 / 8 heads, two workgroups a CU:
+    // 52-63 of 128-2048 34.9 / 34.0, 33.2 / 32.9, 38.0 / 37.2, 39.3 / 38.8; an fp8 cache alike;
+    // 44 and 48 stay whole (33.8, 35.2).  In a mixed launch, where the prefill items
     // fill most gaps, sequences are split at 1024 keys (three items per CU at
     // most) instead, from an excess of 2 MB: 64 decodes of 512-4096 keys and two
     // chunks 143 us unsplit, 113 so, 119 page-balanced (2.4 MB); 100 such decodes

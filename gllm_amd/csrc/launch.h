@@ -48,9 +48,14 @@ constexpr int kPrefillOnlyStages = 4;
 // make at least kTileMinWgs of its workgroups: below that it leaves CUs idle
 // and walks a sequence's keys in one wave each, where the stream kernel splits
 // them over eight.  Measured (stream / tile us, 32 / 8 heads, 2048 cached
-// keys): 64 workgroups (1 x 256 rows) 80 / 234 at D = 64, 134 / 381 at D = 128;
-// 128 (8 x 64) 150 / 220 and 243 / 358; 256 (32 x 32) 348 / 222 and 609 / 372;
-// 512 (8 x 256) 593 / 383 and 1000 / 657.
+// keys), 64, 128, 192, 256 and 512 workgroups (1 x 256, 2 x 256, 3 x 256, 32 x 32 and
+// 8 x 256 rows): fp32 D = 64 88 / 222, 170 / 228, 249 / 241, 348 / 215, 593 / 399; fp32
+// D = 128 152 / 386, 282 / 392, 415 / 395, 698 / 378, 1101 / 747; bf16 D = 96 113 / 303,
+// 212 / 306, 304 / 309, 377 / 293, 795 / 523 (fp16 and an fp8 cache at D = 80 alike); bf16
+// over an fp32 cache, D = 128 126 / 391, 235 / 395, 347 / 395, 596 / 368, 883 / 786; D = 256,
+// 16 / 4 heads, 64, 96, 256 workgroups 203 / 748, 291 / 757, 760 / 764.  Where a tile holds
+// half its columns the line is low: 32 / 32 heads of 80, 12 x 64 rows on 2048 keys (384)
+// 301 / 488.
 constexpr int kStreamCols = 16;
 constexpr int kTileCols = 128;
 constexpr int kTileMinRows = 17;

@@ -10,12 +10,12 @@
 // k and v cast to the cache dtype and stored at slot_mapping[token]
 // (attention.py:156-161), padded rows skipped; q written to q_out.
 //
-// Tiling: one 4-wave workgroup per (128 tokens, one head of D outputs); for
-// large batches at D = 128, one 8-wave workgroup per (256 tokens, two heads)
-// whose waves each take 64 tokens x one head (two row blocks share every W
-// operand read); both launched in XCD-grouped order (qkv_groups).  X and W
-// K-slices of 32 stream HBM/L2 -> LDS with global_load_lds into a 4-stage
-// ring (XOR-swizzled 16-byte chunks: operand reads are bank-conflict free);
+// Tiling: one 4-wave workgroup per (128 tokens, one head of D outputs), in
+// XCD-grouped order (qkv_groups); larger batches take 8-wave tiles of 256 (or
+// 128) tokens x 256 columns (qkv_tile_kernel, below; the line is drawn in
+// launch_qkv_rope_write).  X and W K-slices of 64 (32 where hidden is no
+// multiple of 64) stream HBM/L2 -> LDS with global_load_lds into a ring of 2 (4)
+// stages (XOR-swizzled 16-byte chunks: operand reads are bank-conflict free);
 // each wave computes 32 tokens x D outputs per row block on
 // v_mfma_f32_32x32x16_bf16 (D/32 accumulator blocks).  Output column n of
 // block b is head dim 32b + n, so a RoPE pair (d, d + D/2) sits in blocks b
@@ -1176,9 +1176,11 @@ hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
       else hipLaunchKernelGGL((qkv_rope_write_kernel<64, false, 128, 1, 1, true>), grid, block, 0, st, b);
     }
   } else if (a.head_dim == 128) {
-    // Large batches: 256 tokens x 2 heads per 8-wave workgroup (each wave 64
-    // tokens x one head: two row blocks share every W operand read), in
-    // XCD-grouped order; they need heads that pair within q and within k/v.
+    // Large batches that the 256-column tiles do not take (hidden no multiple of
+    // 64, cache or cos/sin rows off 16 bytes, very long row strides): 256 tokens x 2
+    // heads per 8-wave workgroup (each wave 64 tokens x one head: two row blocks
+    // share every W operand read), in XCD-grouped order; they need heads that pair
+    // within q and within k/v.
     const int64_t tiles2 = (a.num_tokens + 255) / 256;
     if (b.num_q_heads % 2 == 0 && a.num_kv_heads % 2 == 0 && tiles2 * (heads / 2) >= 2 * (int64_t)a.cus) {
       const QKVGroups gr2 = qkv_groups(tiles2, heads / 2, a.cus);

@@ -188,6 +188,7 @@ struct gllm_attn_plan {
   // generic kernels: query rows from which a sequence is tiled (0: none), the
   // largest query length below that
   int32_t tile_min_q = 0, max_stream_q = 0;
+  int64_t stream_rows = 0;       // query rows of the sequences below that
   // page-balanced decode: workgroup w runs segs[seg_ptr[w] .. seg_ptr[w + 1])
   std::vector<DecodeSeg> segs;
   std::vector<int32_t> seg_ptr;
@@ -644,7 +645,7 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
   p->num_seqs = num_seqs; p->Hq = num_q_heads; p->Hkv = num_kv_heads; p->D = head_dim;
   p->bs = block_size; p->dtype = dtype; p->mfma = mfma;
   p->seqs.resize(num_seqs);
-  int64_t row = 0, tile_wgs = 0;
+  int64_t row = 0, all_rows = 0, tile_wgs = 0;
   for (int i = 0; i < num_seqs; ++i) {
     const int32_t ql = query_lens[i], sl = seq_lens[i];
     if (ql < 1 || sl < ql) {
@@ -662,8 +663,11 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
     s.q_len = ql;
     row += ql;
     p->max_q = std::max(p->max_q, ql);
-    if (ql < kTileMinRows) p->max_stream_q = std::max(p->max_stream_q, ql);
-    else tile_wgs += ((int64_t)ql * G + kTileCols - 1) / kTileCols * num_kv_heads;
+    all_rows += ql;
+    if (ql < kTileMinRows) {
+      p->max_stream_q = std::max(p->max_stream_q, ql);
+      p->stream_rows += ql;
+    } else tile_wgs += ((int64_t)ql * G + kTileCols - 1) / kTileCols * num_kv_heads;
   }
   p->total_rows = q_seq_stride > 0 ? (int64_t)num_seqs * q_seq_stride : row;
   if (p->total_rows > INT32_MAX) {
@@ -672,7 +676,10 @@ int gllm_attn_plan_create(gllm_attn_plan** out, const int32_t* query_lens, const
   }
 
   if (tile_wgs >= kTileMinWgs) p->tile_min_q = kTileMinRows;
-  else p->max_stream_q = p->max_q;
+  else {
+    p->max_stream_q = p->max_q;
+    p->stream_rows = all_rows;
+  }
 
   if (mfma) {
     const int cus = device_cus();
@@ -1152,7 +1159,8 @@ static int paged_attention_impl(const gllm_attn_plan* p, const void* q, int64_t 
     a.tile_items = a.items;
     a.n_tile_items = a.n_items;
   }
-  return hip_check(launch_attention_generic(a, false, p->num_seqs, p->max_q, p->max_stream_q, st), "generic attention launch");
+  return hip_check(launch_attention_generic(a, false, p->num_seqs, p->max_q, p->max_stream_q, p->stream_rows, st),
+                   "generic attention launch");
 }
 
 int gllm_paged_attention(const gllm_attn_plan* p, const void* q, int64_t q_row_stride, void* out,
@@ -1213,7 +1221,7 @@ int gllm_attention_dense(const void* q, int64_t q_row_stride, const void* k, int
   hipStream_t st = (hipStream_t)stream;
   if (mfma_dtype(dtype) && (head_dim == 64 || head_dim == 128))
     return hip_check(launch_dense_attention_mfma(a, batch, q_len, st), "dense attention launch");
-  return hip_check(launch_attention_generic(a, true, batch, q_len, q_len, st), "generic dense attention launch");
+  return hip_check(launch_attention_generic(a, true, batch, q_len, q_len, (int64_t)batch * q_len, st), "generic dense attention launch");
 }
 
 }  // extern "C"

@@ -41,7 +41,8 @@ static hipError_t launch_kind(AttnArgs a, bool tile, bool dense, dim3 grid, hipS
   }
 }
 
-hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, hipStream_t st) {
+hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, int64_t stream_rows,
+                                    hipStream_t st) {
   if (B == 0 || max_q == 0) return hipSuccess;
   if (a.head_dim <= 0 || a.head_dim > 256) return hipErrorInvalidValue;
   const int G = a.num_q_heads / a.num_kv_heads;
@@ -62,7 +63,14 @@ hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, in
     if (hipError_t e = launch_kind(a, true, false, g, st); e != hipSuccess) return e;
   }
   if (max_stream_q == 0) return hipSuccess;
-  return launch_kind(a, false, false, grid(max_stream_q, kStreamCols), st);
+  // Where most workgroups are empty (decodes beside a chunk: all but their first)
+  // the column groups are an odd number: at an even stride the working ones all
+  // fell to a few shader engines.  9 decodes and a chunk of 125 rows, bf16 D = 80,
+  // 177 -> 42 us (apart 29 and 22); fp32 D = 64, 11 and two of 24-48 45 -> 22.  Sequences
+  // of like length keep the even stride: two of 39-78 rows 14 -> 18 otherwise.
+  dim3 g = grid(max_stream_q, kStreamCols);
+  if (2 * stream_rows < (int64_t)B * max_stream_q) g.x |= 1;
+  return launch_kind(a, false, false, g, st);
 }
 #endif  // GLLM_GENERIC_DISPATCH
 

@@ -194,6 +194,7 @@ hipError_t launch_paged_attention_mfma(const AttnArgs& a, bool has_prefill, bool
 hipError_t launch_dense_attention_mfma(const AttnArgs& a, int B, int Tq, hipStream_t stream);
 // Generic kernels: max_q the largest query length, max_stream_q the largest of
 // the sequences on the stream kernel (0: every sequence is tiled)
-hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, hipStream_t stream);
+hipError_t launch_attention_generic(AttnArgs a, bool dense, int B, int max_q, int max_stream_q, int64_t stream_rows,
+                                    hipStream_t stream);
 
 }  // namespace gllm

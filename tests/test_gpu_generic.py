@@ -43,6 +43,13 @@ def test_paged(ctx, ql, dtype, kv, D, Hq, Hkv):
     _check(out, oracle_paged(b), f"{dtype} {kv} {D}")
 
 
+@pytest.mark.parametrize("ctx,ql", [([0, 63, 300, 17, 4], [32, 1, 1, 1, 2]),    # 8 column groups at G = 4, odd with one more
+                                    ([5, 0, 40], [1, 45, 1]), ([8, 130, 65], [16, 1, 3])])
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (BF, 80)])
+def test_decodes_beside_a_chunk(ctx, ql, dtype, D):
+    test_paged(ctx, ql, dtype, dtype, D, 32, 8)
+
+
 def test_paged_unaligned_rows():
     """Cache rows at odd element offsets: the element loads of both kernels."""
     for ctx, ql in (FEW, MANY):

@@ -15,7 +15,8 @@
 // 128) tokens x 256 columns (qkv_tile_kernel, below; the line is drawn in
 // launch_qkv_rope_write).  X and W K-slices of 64 (32 where hidden is no
 // multiple of 64) stream HBM/L2 -> LDS with global_load_lds into a ring of 2 (4)
-// stages (XOR-swizzled 16-byte chunks: operand reads are bank-conflict free);
+// stages (XOR-swizzled 16-byte chunks; the counters still show 4 conflict cycles
+// among the 8 of an operand read of 64-wide slices, qkv_tile_kernel's too);
 // each wave computes 32 tokens x D outputs per row block on
 // v_mfma_f32_32x32x16_bf16 (D/32 accumulator blocks).  Output column n of
 // block b is head dim 32b + n, so a RoPE pair (d, d + D/2) sits in blocks b

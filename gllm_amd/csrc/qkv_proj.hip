@@ -1035,24 +1035,25 @@ static QKVTiles qkv_tiles(int64_t n, int ngroups, int cus) {
 // Whether a prompt batch's tiles are ahead of three library GEMMs and the RoPE +
 // KV write kernel.  Both run 256 x 256 tiles in rounds of one per CU, so each
 // side's time goes with its rounds: the tiles' over all columns together, the
-// library's over q, k and v by themselves, a GEMM of less than half (a quarter)
-// of a round taking 0.8 (0.4) of one in smaller tiles.  The library's rounds are
-// shorter by an eighth (hidden 4096: 93-105 us against 104-117), and a round of
-// the tiles' half tiles measures 0.62 here, so the tiles go first from 1.12 of
-// their rounds on.  Measured over 52 sizes of 3,072-19,700 tokens, us, library /
-// tiles (library rounds / tiles'): 32 / 8 heads of 128, hidden 4096: 4,100 tokens
-// 252 / 209 (1.40), 12,000 662 / 504 (1.08), 12,288 492 / 540 (1.03), 13,677 566 / 627
-// (1.02), 16,384 628 / 694 (1.00), 16,390 960 / 721 (1.38), 19,679 950 / 847 (1.19);
-// hidden 3072, 24 / 8 heads: 3,244 125 / 146 (0.97), 9,768 295 / 328 (1.04); 32 / 8
-// heads of 64, hidden 2048: 4,096 78 / 59 (1.81), 5,377 98 / 103 (0.97).  Of 292
-// points the rule gives 224 to the tiles, 223 of them no slower than 1% (17,906
-// tokens 763 / 793), and most of the others within 10% of a draw.
-constexpr double kLibraryRound = 1.12, kHalfRoundAhead = 0.62;
+// library's over q, k and v by themselves, a GEMM of less than half (a quarter, an
+// eighth) of a round taking 0.8 (0.4, 0.3) of one in smaller tiles.  The library's rounds are
+// shorter by a twelfth (hidden 4096: 93-105 us against 104-117), and a round of
+// the tiles' half tiles measures 0.62 here, so the tiles go first from 1.08 of
+// their rounds on.  Measured over 50 sizes of 3,073-19,700 tokens, us, library /
+// tiles (library rounds / tiles'): 32 / 8 heads of 128, hidden 4096: 3,500 tokens 184 /
+// 170 (1.11), 4,100 252 / 209 (1.40), 12,000 662 / 504 (1.08), 12,288 492 / 540 (1.03), 13,677
+// 566 / 627 (1.02), 16,384 628 / 694 (1.00), 16,390 960 / 721 (1.38), 19,679 950 / 847 (1.19);
+// hidden 3072, 24 / 8 heads: 3,950 143 / 131 (1.11), 9,868 284 / 289 (1.10); 32 / 8
+// heads of 64, hidden 2048: 4,096 75 / 54 (1.4), 5,377 99 / 84 (1.11); 32 / 2 heads of 128,
+// hidden 4096: 3,300 142 / 110 (1.6), 4,096 151 / 161 (0.99).  Over 300 points
+// of six layers the choice is 1.174x the library alone (1.181x with the better side
+// each time), weights from HBM, 5 of them more than 2% behind it.
+constexpr double kLibraryRound = 1.08, kHalfRoundAhead = 0.62;
 bool qkv_tiles_ahead(int64_t n, int q_cols, int kv_cols, int cus) {
   const int64_t tiles = (n + 255) / 256;
   const auto gemm = [&](int cols) {
     const double r = (double)(tiles * cols) / 256 / cus;
-    return cols == 0 ? 0.0 : r <= 0.25 ? 0.4 : r <= 0.5 ? 0.8 : std::ceil(r);
+    return cols == 0 ? 0.0 : r <= 0.125 ? 0.3 : r <= 0.25 ? 0.4 : r <= 0.5 ? 0.8 : std::ceil(r);
   };
   const int ngroups = (q_cols + 2 * kv_cols) / kTCols;
   if (ngroups <= 0) return false;
@@ -1128,22 +1129,25 @@ hipError_t launch_qkv_rope_write(const QKVArgs& a, hipStream_t st) {
     const int ngroups = heads / hp;
     const QKVTiles t = qkv_tiles(a.num_tokens, ngroups, a.cus);
     // The 128-token x one-head tiles keep a batch that they finish in one go, two per
-    // CU on the fullest XCD (super-groups are dealt out whole): always at head dim 64,
-    // at 128 unless they are so many per CU that their starts weigh more: over 1 up to
-    // hidden 2560, from 1.5 at 4096-4608; between and above they stay ahead or even.
+    // CU on the fullest XCD (super-groups are dealt out whole): always at head dim 64;
+    // at 128 up to hidden 4608 only with at most one per CU, above it always.  With more
+    // than one, weights decide: from HBM, as between the layers of a model, the small
+    // tiles' many workgroups fetch them sooner, from the Infinity Cache (256 MB) the
+    // large ones' fewer operand reads win; the line goes with the smaller loss.
     // Measured over 20 layers, 300-3,071 tokens (us, those / these): head dim 64: 48 heads,
     // hidden 2048, 1,024 tokens 29 / 33; 64 heads, 3072, 1,024 / 1,100 (not one go) 45 / 62,
-    // 72 / 60.  Head dim 128: 32 heads, 2048, 1,024 / 1,100 (1.0, 1.1 per CU) 32 / 34, 41 / 34;
-    // 28 heads, 2560, 1,300 (1.2) 49 / 42; 40 heads, 3072, 900 / 1,300 / 1,536 (1.25, 1.7, 1.9)
-    // 58 / 62, 59 / 62, 66 / 64; 40 heads, 4096, 1,300 (1.7) 79 / 73; 48 heads, 4096, 700 / 900 /
-    // 1,300 (1.1, 1.5, not one go) 71 / 73, 80 / 73, 118 / 96; 56 heads, 5120, 700 / 1,024
-    // (1.3, 1.75) 86 / 103, 98 / 106; 64 heads, 6144, 700 / 1,024 (1.5, 2.0) 101 / 119, 115 / 117;
-    // 80 heads, 8192, 512 / 700 (1.25, not one go) 145 / 153, 230 / 152.
+    // 72 / 60.  Head dim 128, weights from HBM (from the cache): 32 heads, 2048, 1,024 / 1,100
+    // (1.0, 1.1 per CU) 32 / 34, 41 / 34; 28 heads, 2560, 1,300 (1.2) 49 / 42; 40 heads, 3072, 900 /
+    // 1,300 (1.25, 1.7) 58 / 62, 59 / 62 (58 / 47, 61 / 50); 40 heads, 4096, 900 / 1,300 (1.25, 1.7)
+    // 70 / 72, 79 / 73 (73 / 56, 62 / 62 both these); 48 heads, 4096, 700 / 830 / 900 (1.1, 1.3,
+    // 1.5) 71 / 73, 75 / 73, 80 / 73 (72 / 60, 76 / 61, 76 / 62); 44 heads, 4608, 700 / 900 (1.0, 1.4)
+    // 76 / 85, 87 / 86 (79 / 63, 88 / 63); 56 heads, 5120, 700 / 1,024 (1.3, 1.75) 86 / 103, 98 / 106
+    // (88 / 74, 101 / 79); 64 heads, 6144, 700 / 1,024 (1.5, 2.0) 101 / 119, 115 / 117 (101 / 84,
+    // 116 / 96); 80 heads, 8192, 512 / 700 (1.25, not one go)
+    // 145 / 153, 230 / 152.
     const QKVGroups gr = qkv_groups(tiles, heads, a.cus);
     const bool one_go = (gr.nsg + kXcds - 1) / kXcds * gr.gt * gr.gh <= 2 * (int64_t)a.cus / kXcds;
-    const int64_t small = tiles * heads;
-    const bool ahead = a.hidden <= 2560 ? small > a.cus : a.hidden >= 4096 && a.hidden <= 4608 && 2 * small >= 3 * a.cus;
-    if (!one_go || (a.head_dim == 128 && ahead)) {
+    if (!one_go || (a.head_dim == 128 && a.hidden <= 4608 && tiles * heads > a.cus)) {
       const auto wgs_of = [&](int64_t tiles) { return (tiles * ngroups + kXcds - 1) / kXcds * kXcds; };
       b.full_tiles = (int32_t)t.full;
       b.half_tiles = (int32_t)t.half;

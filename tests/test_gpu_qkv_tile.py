@@ -59,7 +59,7 @@ def test_short_last_round_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad):
 @pytest.mark.parametrize("n,hidden,Hq,Hkv,D,kv,rot,pad", [
     (640, 64, 32, 8, 128, BF, True, False), (641, 64, 32, 8, 128, BF, True, False),     # one small tile per CU, over it
     (1281, 64, 32, 8, 64, F8, True, False), (1409, 64, 32, 8, 64, BF, True, False),     # two per CU at head dim 64, over it
-    (1024, 4096, 24, 8, 128, BF, False, False), (1153, 4096, 24, 8, 128, BF, True, False),   # 1.25 and 1.4 per CU
-    (1281, 4096, 24, 8, 128, F8, True, False)])                                            # 1.7
+    (768, 4096, 24, 8, 128, BF, False, False), (769, 4096, 24, 8, 128, BF, True, False),   # 0.94 and 1.1 per CU
+    (1281, 4096, 24, 8, 128, F8, True, False), (1024, 5120, 24, 8, 128, BF, True, False)])   # 1.7; 1.25 of a wider layer
 def test_both_sides_of_the_line_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad):
     test_tile256_bit_exact(n, hidden, Hq, Hkv, D, kv, rot, pad)

@@ -81,8 +81,8 @@ def test_qkv_split_fits_the_noalloc_scratch(hidden, heads):
 
 @pytest.mark.parametrize("Hq,Hkv,D,behind,ahead", [
     (32, 8, 128, [3984, 4096, 12286, 12288, 13627, 15718, 15884, 16384], [4100, 5282, 8200, 10362, 16390, 17099, 19679]),
-    (24, 8, 128, [3244, 9768, 9868, 15748, 16384], [3072, 3148, 5377, 6043, 16390, 18608]),
-    (32, 8, 64, [5377], [3072, 4096, 5186, 9768, 16384, 19352]),
+    (24, 8, 128, [15748, 16384], [3072, 3148, 3244, 5377, 6043, 16390, 18608]),
+    (32, 8, 64, [], [3072, 4096, 5186, 5377, 9768, 16384, 19352]),
     (32, 2, 128, [3798, 4096, 7397, 16384], [3148, 4100, 8436, 9003, 19352]),
     (4, 4, 64, [], [3072, 8192, 19679]), (2, 2, 128, [], [3072, 6000, 19679])])
 def test_prompt_projections_where_the_library_is_ahead(Hq, Hkv, D, behind, ahead):
